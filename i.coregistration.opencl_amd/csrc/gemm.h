@@ -1,6 +1,6 @@
 /* SPDX-License-Identifier: Unlicense */
 
-/* The fp32 MFMA GEMM kernel family behind ops_gemm, ops_linear,
+/* The float32 GEMM kernel family behind ops_gemm, ops_linear,
  * ops_conv1x1 and the one-group ops_conv2d (implicit GEMM). */
 
 #ifndef ICOREG_GEMM_H
@@ -47,9 +47,9 @@ struct gemm_args {
      * table row r % rnpos of rope for output row r). */
     const float2 *rope;
     int rcols, rd, rnpos;
-    /* Main kernel, one batch: tiles nfull.. are cut into split pieces
-     * over K whose partial sums go to part (4096 floats a piece) and are
-     * added by a second kernel (gemm_split_floats; split <= 1: none). */
+    /* Main kernels, one batch: tiles nfull.. are cut into split pieces
+     * over K whose partial sums go to part (gemm_part_floats floats;
+     * NULL: no tile is cut) and are added by a second kernel. */
     int nfull, split;
     float *part;
 };
@@ -63,9 +63,15 @@ bool gemm_shape_ok(const gemm_args &g, int bmode);
 void gemm_launch(const gemm_args &g, int bmode, int nb, bool va, bool vb,
                  int cus, hipStream_t s);
 
-/* Floats of part that gemm_launch's main kernel needs for g (0: it
- * runs without pieces). */
-size_t gemm_split_floats(const gemm_args &g, int bmode, int nb, bool va, bool vb, int cus);
+/* Floats of part that gemm_launch's kernel for g needs (0: it runs without
+ * pieces). */
+size_t gemm_part_floats(const gemm_args &g, int bmode, int nb, bool va, bool vb, int cus);
+
+/* gemm_launch and gemm_part_floats for the products of the bf16
+ * instructions (gemm_split.hip). */
+void gemm_split_launch(const gemm_args &g, int bmode, int nb, bool va, bool vb, int cus,
+                       hipStream_t s);
+size_t gemm_split_floats(const gemm_args &g, int bmode, int nb, int cus);
 
 /* True if gemm_launch would run g on the small-product kernel. */
 bool gemm_smallk_ok(const gemm_args &g, int bmode, int nb, bool va, bool vb, int cus);

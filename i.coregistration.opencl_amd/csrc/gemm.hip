@@ -1,6 +1,8 @@
 /* SPDX-License-Identifier: Unlicense */
 
-/* fp32 GEMM on the CDNA4 matrix cores: C = act(alpha A op(B) + bias) + R.
+/* fp32 GEMM on the CDNA4 fp32 matrix instructions: C = act(alpha A op(B) +
+ * bias) + R. Products of K up to GEMM_SPLIT_K (gemm_launch); longer ones run
+ * in gemm_split.hip.
  *
  * The contract is the reference's gemm / gemm_big (ops.cl:39-284 of
  * i.coregistration.opencl): batched over nb = nb0 * nb1 with two batch
@@ -33,120 +35,12 @@
 #include <algorithm>
 #include <hip/hip_runtime.h>
 
-#include "act.h"
-#include "bilinear.h"
-#include "gemm.h"
-
-typedef float floatx16 __attribute__((ext_vector_type(16)));
+#include "gemm_dev.h"
 
 #define GEMM_PAD 4
 
-/* Offset past the end of every window: the load reads 0. */
-#define GEMM_OOB 0x80000000u
-/* gfx9 s_waitcnt immediate: vmcnt(0), expcnt and lgkmcnt not waited on. */
-#define GEMM_WAIT_VM0 0x0F70
-
-/* Word 3 of a raw buffer resource on gfx9-family parts: 32-bit data. */
-#define GEMM_RSRC_FLAGS 0x00020000
-
-/* Buffer window of `bytes` bytes from p: loads at byte offsets at or past
- * its end return 0. */
-static __device__ __forceinline__ __amdgpu_buffer_rsrc_t
-gemm_rsrc(const float *p, long long bytes)
-{
-    return __builtin_amdgcn_make_buffer_rsrc((void *)p, (short)0,
-                                             (int)(unsigned)bytes,
-                                             GEMM_RSRC_FLAGS);
-}
-
-/* Four consecutive floats at byte offset off of window r: one 16-byte
- * load (VEC: the four are either all inside the window or all past its
- * end), else four 4-byte loads. */
-template <bool VEC>
-__device__ __forceinline__ float4 gemm_load4(__amdgpu_buffer_rsrc_t r,
-                                             unsigned off)
-{
-    if (VEC)
-        return __builtin_bit_cast(
-            float4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0));
-    float4 v;
-
-    v.x = __builtin_bit_cast(
-        float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, 0));
-    v.y = __builtin_bit_cast(
-        float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off + 4, 0, 0));
-    v.z = __builtin_bit_cast(
-        float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off + 8, 0, 0));
-    v.w = __builtin_bit_cast(
-        float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off + 12, 0, 0));
-    return v;
-}
-
-/* Components i of v with lo + i >= hi set to 0. */
-__device__ __forceinline__ float4 mask4(float4 v, int lo, int hi)
-{
-    v.x = lo < hi ? v.x : 0.0f;
-    v.y = lo + 1 < hi ? v.y : 0.0f;
-    v.z = lo + 2 < hi ? v.z : 0.0f;
-    v.w = lo + 3 < hi ? v.w : 0.0f;
-    return v;
-}
-
 /* Most pieces a cut GEMM tile is split into. */
 #define GEMM_MAX_SPLIT 8
-
-/* Output tile of linear block id L among T tiles: blocks are dealt to
- * the 8 XCDs round-robin (L % 8), so give XCD x the x-th contiguous
- * band of tiles. A bijection of 0..T-1. */
-__device__ __forceinline__ int xcd_tile(int L, int T)
-{
-    const int q = T >> 3, rem = T & 7, x = L & 7, idx = L >> 3;
-
-    return (x < rem ? x * (q + 1) : rem * (q + 1) + (x - rem) * q) + idx;
-}
-
-/* C = act(alpha acc + bias) + R for the TM x TN 32 x 32 tiles of a wave
- * whose block of C starts at (r0, c0), batch (b0, b1). Register r of a
- * tile holds row (r / 4) * 8 + (lane / 32) * 4 + r % 4, column lane % 32. */
-template <int TM, int TN>
-__device__ __forceinline__ void gemm_epilogue(const gemm_args &g, const floatx16 (&acc)[TM][TN],
-                                              long long b0, long long b1, int r0, int c0,
-                                              int lane)
-{
-    float *C = g.C + b0 * g.sc0 + b1 * g.sc1;
-    const float *R =
-        g.R ? (g.rup ? g.R + b0 * g.rs0 : g.R + b0 * g.sc0 + b1 * g.sc1) : nullptr;
-
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++) {
-            const int col = c0 + j * 32 + (lane & 31);
-            const int ry = g.rup ? col / g.rwo : 0, rx = g.rup ? col - ry * g.rwo : 0;
-
-            if (col >= g.N)
-                continue;
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int row = r0 + i * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
-                float v;
-
-                if (row >= g.M)
-                    continue;
-                v = g.alpha * acc[i][j][r];
-                if (g.bias)
-                    v += g.bias[g.biasrow ? row : col];
-                if (R && g.rpre)
-                    v += bl_up(R + (long long)row * g.rh * g.rw, g.rh, g.rw, g.rsc, ry, rx);
-                v = icoreg_act(v, g.act, g.slope);
-                if (R && !g.rpre)
-                    v += g.rup ? bl_up(R + (long long)row * g.rh * g.rw, g.rh, g.rw, g.rsc, ry,
-                                       rx)
-                               : R[(long long)row * g.ldc + col];
-                C[(long long)row * g.ldc + col] = v;
-            }
-        }
-}
 
 /* BM x BN output tile, BK slice, WGM x WGN waves (each a
  * BM / WGM x BN / WGN block of 32 x 32 MFMA tiles). */
@@ -1019,10 +913,22 @@ static bool gemm_plan(const gemm_args &g, int bmode, int nb, int cus, int &nfull
     return split > 1;
 }
 
-size_t gemm_split_floats(const gemm_args &g, int bmode, int nb, bool va, bool vb, int cus)
+/* Products that run on the bf16 instructions (gemm_split.hip): sums of
+ * more than GEMM_SPLIT_K products. Alone the shorter ones gain too, most of
+ * them under a fifth (ELoFTR's K = 128 .. 512: 1.14 -> 1.04 ms a pair), but
+ * the bf16 instructions draw more power than the fp32 ones and the kernels
+ * around them then run at a lower clock (ELoFTR's fp32 convolutions 8 - 10 %
+ * slower: 4.12 -> 4.23 ms a pair in all). */
+#define GEMM_SPLIT_K 512
+
+static bool gemm_split_ok(const gemm_args &g) { return g.K > GEMM_SPLIT_K; }
+
+size_t gemm_part_floats(const gemm_args &g, int bmode, int nb, bool va, bool vb, int cus)
 {
     int nfull, split;
 
+    if (gemm_split_ok(g))
+        return gemm_split_floats(g, bmode, nb, cus);
     va = va && g.K % 4 == 0;
     vb = vb && (bmode == GEMM_B_KN ? g.N % 4 == 0 : g.K % 4 == 0);
     if (gemm_smallk_ok(g, bmode, nb, va, vb, cus) || gemm_dma_ok(g, bmode, va, vb) ||
@@ -1039,6 +945,10 @@ void gemm_launch(const gemm_args &g, int bmode, int nb, bool va, bool vb,
      * K x N) a multiple of 4. */
     va = va && g.K % 4 == 0;
     vb = vb && (bmode == GEMM_B_KN ? g.N % 4 == 0 : g.K % 4 == 0);
+    if (gemm_split_ok(g)) {
+        gemm_split_launch(g, bmode, nb, va, vb, cus, s);
+        return;
+    }
     /* 64 x 64 tiles, 4 waves, BK = 16 at every shape: 17 KB of LDS and
      * few registers keep up to 8 waves per SIMD in flight. In isolated
      * sweeps 64 x 128 (8 waves, BK = 32) and 128 x 128 (16 waves) tiles

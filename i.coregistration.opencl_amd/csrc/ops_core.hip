@@ -41,6 +41,18 @@ cl_mem scratch_get(struct ops *o, size_t bytes)
     return o->scratch;
 }
 
+/* scratch_get, or NULL where it would have to grow while the stream is
+ * recorded into a graph (nothing can be allocated then). */
+static cl_mem scratch_or_null(struct ops *o, size_t bytes)
+{
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+
+    if (bytes <= o->scratch_bytes && o->scratch)
+        return o->scratch;
+    hip_check(hipStreamIsCapturing(stream_of(o->ocl), &st), "hipStreamIsCapturing");
+    return st == hipStreamCaptureStatusNone ? scratch_get(o, bytes) : NULL;
+}
+
 } // namespace icoreg
 
 extern "C" void ops_free(struct ops *o)
@@ -188,10 +200,10 @@ extern "C" void ops_gemm(struct ops *o, int M, int N, int K, struct opnd A,
         gemm_args g = gemm_make(op, M, N, K, A, B, transb, C, nb, nb1, bias, biasrow, R, roff,
                                 alpha, act, slope);
         /* Partial sums of cut tiles, when the grid leaves CUs uneven. */
-        const size_t pf = gemm_split_floats(g, bmode, nb, vec_ok(A), vec_ok(B), o->ocl->cu_count);
+        const size_t pf = gemm_part_floats(g, bmode, nb, vec_ok(A), vec_ok(B), o->ocl->cu_count);
 
         if (pf)
-            g.part = fptr(scratch_get(o, pf * sizeof(float)));
+            g.part = fptr(scratch_or_null(o, pf * sizeof(float)));
         prof_scope ps(o->ocl, "gemm");
         gemm_launch(g, bmode, nb, vec_ok(A), vec_ok(B), o->ocl->cu_count, stream_of(o->ocl));
         launch_check("gemm");

@@ -1,0 +1,114 @@
+# SPDX-License-Identifier: Unlicense
+"""GPU: ops_gemm on the bf16 matrix instructions (products of more than 512
+terms) against float64 sums, at the edges of its tiles and cuts.
+
+Bound: a value's six kept bf16 products leave out less than 2^-25 of |a b|;
+the matrix core adds groups of eight k, so K / 8 additions round by 2^-24 of
+a partial sum that sum |a b| bounds, and a group's alignment drops at most
+8 * 2^-24 of its largest product: 2^-24 (K / 8 + 16) sum |a b| in all, and
+the float32 epilogue's own 2^-24 a step."""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+U = 2.0 ** -24
+
+# (M, N, K, transb, nb, act, residual, biasrow); act 0 none, 2 ReLU, 3 leaky.
+SHAPES = [
+    # One output, one row, one column; K just past the rule, K % 32 != 0.
+    (1, 1, 513, 1, 1, 0, 0, 0),
+    (1, 70, 516, 0, 1, 0, 1, 1),
+    (70, 1, 544, 1, 1, 3, 0, 0),
+    # Around one and two 64- and 128-row tiles, aligned and not.
+    (64, 64, 544, 1, 1, 0, 0, 0),
+    (65, 63, 1023, 1, 1, 2, 0, 1),
+    (128, 128, 576, 0, 2, 0, 1, 0),
+    (129, 127, 577, 0, 1, 3, 0, 1),
+    (127, 260, 1140, 0, 3, 2, 1, 0),
+    # Every tile cut over K (few tiles, long K); the last piece shorter.
+    (100, 90, 4100, 1, 1, 0, 1, 0),
+    (96, 200, 2052, 0, 1, 3, 0, 1),
+    # 288 tiles of 128 x 128: 256 whole, 32 cut.
+    (2304, 2000, 1024, 1, 1, 0, 1, 0),
+]
+
+
+def run(dev, ic, a, b, shape, alpha, bias, r):
+    M, N, K, transb, nb, act, residual, biasrow = shape
+    ldb = K if transb else N
+    A, B, Bi = dev.upload(a), dev.upload(b), dev.upload(bias)
+    out = dev.upload(r)
+    dev.api.ops_gemm(dev.po, M, N, K, ic.bmat(A, 0, K, M * K, 0), ic.bmat(B, 0, ldb, N * K, 0),
+                     transb, ic.bmat(out, 0, N, M * N, 0), nb, 1, ic.mem(Bi), biasrow,
+                     ic.mem(out) if residual else None, 0, alpha, act, 0.1)
+    return dev.read(out, nb * M * N).reshape(nb, M, N)
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=[str(s) for s in SHAPES])
+def test_edges(shape, dev, ic):
+    M, N, K, transb, nb, act, residual, biasrow = shape
+    print(f"[gemm split] {shape}", flush=True)
+    rng = np.random.default_rng(M + 3 * N + K)
+    a = rng.standard_normal((nb, M, K)).astype(np.float32)
+    b = rng.standard_normal((nb, N, K) if transb else (nb, K, N)).astype(np.float32)
+    bias = rng.uniform(-1, 1, M if biasrow else N).astype(np.float32)
+    r = rng.uniform(-1, 1, (nb, M, N)).astype(np.float32)
+    got = run(dev, ic, a, b, shape, 0.5, bias, r)
+    bt = np.swapaxes(b, 1, 2) if transb else b
+    v = 0.5 * (a.astype(np.float64) @ bt.astype(np.float64))
+    v += bias[:, None] if biasrow else bias
+    if act:
+        v = np.where(v >= 0, v, (0.0 if act == 2 else 0.1) * v)
+    if residual:
+        v += r
+    size = 0.5 * (np.abs(a).astype(np.float64) @ np.abs(bt).astype(np.float64)) + 2
+    worst = np.max(np.abs(got - v) / (U * ((K / 8 + 16) * size + 4 * np.abs(v))))
+    print(f"[gemm split] worst {worst:.3f} of the bound", flush=True)
+    assert worst <= 1
+
+
+@pytest.mark.parametrize("transb", [0, 1])
+def test_rows_that_are_not_finite(transb, dev, ic):
+    """Infinities, NaN and values that round to bf16 infinity come out as
+    float32 products give them, and leave the other rows alone."""
+    M, N, K = 200, 150, 600
+    rng = np.random.default_rng(11)
+    a = rng.standard_normal((1, M, K)).astype(np.float32)
+    b = rng.standard_normal((1, N, K) if transb else (1, K, N)).astype(np.float32)
+    a[0, 5, 17] = np.inf
+    a[0, 77, 599] = -np.inf
+    a[0, 130, 0] = np.nan
+    a[0, 190] = 0
+    a[0, 190, 3] = 3.4e38  # above the largest bf16
+    bt = np.swapaxes(b, 1, 2) if transb else b
+    bt[0, 17, 9] = 0  # inf * 0
+    with np.errstate(invalid="ignore"):
+        v = (a.astype(np.float64) @ bt.astype(np.float64))[0]
+    with np.errstate(over="ignore"):
+        want = v.astype(np.float32)
+    got = run(dev, ic, a, b, (M, N, K, transb, 1, 0, 0, 0), 1.0, np.zeros(N, np.float32),
+              np.zeros((1, M, N), np.float32))[0]
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    fine = np.isfinite(want)
+    rows = np.delete(np.arange(M), [5, 77, 130])
+    assert fine[190].any() and np.all(fine[np.delete(rows, rows.searchsorted(190))])
+    size = np.abs(a[0, rows]).astype(np.float64) @ np.abs(bt[0]).astype(np.float64)
+    off = np.where(fine[rows], np.abs(got[rows] - v[rows]), 0)
+    assert np.all(off <= U * (K / 2 + 16) * size)
+
+
+def test_sums_of_squares_are_not_biased(dev, ic):
+    """The Gram diagonal: every term positive, so what the small products
+    lose would show as a shift of the mean (it must stay below half a unit
+    in the last place)."""
+    n, K = 256, 1024
+    x = np.random.default_rng(3).standard_normal((1, n, K)).astype(np.float32)
+    g = run(dev, ic, x, x, (n, n, K, 1, 1, 0, 0, 0), 1.0, np.zeros(n, np.float32),
+            np.zeros((1, n, n), np.float32))[0]
+    want = np.sum(x[0].astype(np.float64) ** 2, 1)
+    shift = np.mean(np.diag(g) / want - 1)
+    print(f"[gemm split] mean shift {shift:.2e}", flush=True)
+    assert abs(shift) <= U / 2
