@@ -37,12 +37,28 @@ bool conv_direct_supported(int kh, int kw, int sy, int sx, int dy, int dx,
  * offsets (per-image input and the weights below 2 GiB). */
 bool conv_direct_fits(long long in_floats, long long w_floats);
 
-/* Bytes of the partial sums conv_direct_launch needs for a (0: none);
- * the caller passes that much memory as a.part. */
+/* Bytes of work memory conv_direct_launch needs for a (filters in operand
+ * order and partial sums; 0: none); the caller passes that much as a.part,
+ * or NULL for the kernels that need none. */
 size_t conv_direct_part_bytes(const conv_args &a, int ks, int stride, int nb, int cus);
 
 void conv_direct_launch(const conv_args &a, int ks, int stride, int nb,
                         int cus, hipStream_t s);
+
+/* The direct 5 x 5 convolution, stride 1, on the bf16 matrix instructions
+ * (conv_split.hip): channels a block, tile width, pieces over the input
+ * channels; ok: it takes the shape, and is the faster kernel for it. */
+struct conv_split_plan {
+    int bm, tw, split;
+    bool ok;
+};
+conv_split_plan conv_split_choose(const conv_args &a, int ks, int st, int nb, int cus);
+/* Bytes of the filters of K x C channels in that kernel's operand order. */
+size_t conv_split_weight_bytes(int K, int C);
+/* The convolution of a (a.split = p.split, a.part set where it is > 1),
+ * its filters laid out in wp first. */
+void conv_split_launch(const conv_args &a, const conv_split_plan &p, void *wp, int nb,
+                       hipStream_t s);
 
 /* Winograd F(2 x 2, 3 x 3) path (conv_wino.hip): 3 x 3, stride 1,
  * padding 1, one group, K % 4 == 0, at least 32 channels in and out, an

@@ -659,13 +659,40 @@ static direct_plan plan_direct(const conv_args &a, int ks, int nb, int cus)
     return p;
 }
 
+/* a's main channels for the bf16 kernel: all but the last 1 .. FK_MAXK past
+ * a multiple of its 64, which go to the few-channel kernel. */
+static conv_args split_main(const conv_args &a, int ks)
+{
+    const int rem = a.K % 64;
+    conv_args m = a;
+
+    if (a.K > 64 && rem <= FK_MAXK && a.C <= FK_MAXC &&
+        (long long)rem * a.C * ks * ks <= FK_MAXW)
+        m.K = a.K - rem;
+    return m;
+}
+
+/* Bytes of the bf16 kernel's filters, before the partial sums. */
+static size_t split_filter_bytes(const conv_args &m)
+{
+    return (conv_split_weight_bytes(m.K, m.C) + 255) & ~(size_t)255;
+}
+
 size_t conv_direct_part_bytes(const conv_args &a, int ks, int stride, int nb, int cus)
 {
     if (a.C == 1 && !a.mean && a.K <= C1_MAXK && a.K * ks * ks <= C1_MAXW)
         return 0;
-    const direct_plan p = plan_direct(a, ks, nb, cus);
+    const conv_args m = split_main(a, ks);
+    const conv_split_plan sp = conv_split_choose(m, ks, stride, nb, cus);
+    direct_plan p = plan_direct(a, ks, nb, cus);
+    size_t fewk = 0, filters = 0;
+
+    if (sp.ok) {
+        p.kmain = m.K;
+        p.split = sp.split;
+        filters = split_filter_bytes(m);
+    }
     const size_t main = p.split > 1 ? (size_t)p.split * nb * p.kmain * a.Ho * a.Wo : 0;
-    size_t fewk = 0;
 
     if (p.kmain < a.K) {
         /* The few-channel kernel runs after the main one's pieces are
@@ -676,7 +703,7 @@ size_t conv_direct_part_bytes(const conv_args &a, int ks, int stride, int nb, in
         if (split > 1)
             fewk = (size_t)split * nb * (a.K - p.kmain) * a.Ho * a.Wo;
     }
-    return std::max(main, fewk) * sizeof(float);
+    return filters + std::max(main, fewk) * sizeof(float);
 }
 
 template <int KS, int ST, int BM, int TW, int NJ>
@@ -705,7 +732,27 @@ template <int KS, int ST>
 static void launch_ks(const conv_args &a, int nb, int cus, hipStream_t s)
 {
     constexpr int NJ = KS == 3 ? 1 : 2;
-    const direct_plan p = plan_direct(a, KS, nb, cus);
+    const conv_args m = split_main(a, KS);
+    const conv_split_plan sp = conv_split_choose(m, KS, ST, nb, cus);
+    direct_plan p = plan_direct(a, KS, nb, cus);
+
+    if (sp.ok && a.part) {
+        /* Filters, then the partial sums. */
+        conv_args b = a, c = m;
+
+        b.part = c.part = (float *)((char *)a.part + split_filter_bytes(m));
+        c.split = sp.split;
+        conv_split_launch(c, sp, a.part, nb, s);
+        if (sp.split > 1)
+            hipLaunchKernelGGL(conv_pieces_kernel,
+                               dim3((unsigned)(((long long)m.K * a.Ho * a.Wo + 255) / 256), nb),
+                               dim3(256), 0, s, c, nb);
+        if (m.K < a.K)
+            launch_fewk<KS, ST>(b, m.K, a.K - m.K, nb, cus, s);
+        return;
+    }
+    if (!a.part)
+        p.split = 1;
 
     if (p.bm == 128) {
         if (p.tw == 16)

@@ -602,7 +602,7 @@ static void conv_impl(struct ops *o, int nb, cl_mem in, long long in_stride,
             const size_t pb = conv_direct_part_bytes(a, g->kh, g->sy, nb, o->ocl->cu_count);
 
             if (pb)
-                a.part = fptr(scratch_get(o, pb));
+                a.part = fptr(scratch_or_null(o, pb));
         }
         prof_scope ps(o->ocl, "conv_direct");
         conv_direct_launch(a, g->kh, g->sy, nb, o->ocl->cu_count,

@@ -1,0 +1,92 @@
+# SPDX-License-Identifier: Unlicense
+"""GPU: 5 x 5 convolutions on the bf16 matrix instructions (at least 16
+channels in, 32 out and 96 blocks of 64 channels x 256 pixels) against
+torch's float64 convolution, at the edges of their blocks.
+
+Bound: as for the products of tests/test_gemm_split_gpu.py, 2^-24 (n / 8 +
+16) sum |w x| over the n = 25 C terms, plus the input normalisation's
+rounding (three float32 steps a value, 3 * 2^-24 |w x|)."""
+
+import numpy as np
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+
+U = 2.0 ** -24
+# (images, C, K, H, W, pad, norm, act); act 0 none, 2 ReLU.
+CASES = [
+    (1, 16, 32, 160, 160, 2, 1, 0),     # one slice of channels, half a block of outputs
+    (1, 17, 64, 161, 175, 2, 0, 2),     # a slice with one channel, ragged tiles
+    (1, 33, 65, 97, 190, 2, 1, 0),      # 64 channels and one on the few-channel kernel
+    (2, 20, 150, 60, 127, 2, 1, 2),     # second block of 128 partly empty, pairs
+    (1, 48, 128, 97, 130, 0, 0, 0),     # no padding, pieces over the channels
+    (1, 100, 72, 113, 129, 4, 1, 0),    # padding past the window's half, pieces, K = 64 + 8
+    (2, 40, 200, 67, 65, 1, 1, 2),
+]
+
+
+def tensors(c, seed):
+    n, C, K, H, W, pad, norm, act = c
+    rng = np.random.default_rng(seed)
+    x = rng.standard_normal((n, C, H, W)).astype(np.float32)
+    w = (rng.standard_normal((K, C, 5, 5)) * (2 / (25 * C)) ** 0.5).astype(np.float32)
+    b = rng.uniform(-0.1, 0.1, K).astype(np.float32)
+    v = [rng.uniform(lo, hi, C).astype(np.float32) for lo, hi in ((-0.2, 0.2), (0.8, 1.25), (0.1, 0.3))]
+    return x, w, b, (v if norm else None)
+
+
+def run(dev, ic, c, x, w, b, v):
+    n, C, K, H, W, pad, norm, act = c
+    ho, wo = H + 2 * pad - 4, W + 2 * pad - 4
+    X, Wt, B = dev.upload(x), dev.upload(w), dev.upload(b)
+    V = [dev.upload(t) for t in v] if v else [None] * 3
+    out = dev.zeros(n * K * ho * wo)
+    g = ic.geom(5, 5, 1, 1, pad, pad, 1, 1, 1)
+    dev.api.ops_conv2d_batch(dev.po, n, X.mem, C * H * W, C, H, W, Wt.mem, B.mem, K, ic.C.byref(g),
+                             *(ic.mem(t) for t in V), act, 0.0, out.mem, K * ho * wo)
+    return dev.read(out).reshape(n, K, ho, wo)
+
+
+def want(c, x, w, b, v):
+    n, C, K, H, W, pad, norm, act = c
+    t = torch.from_numpy(x).double()
+    if v:
+        m, r, a = (torch.from_numpy(q).double()[:, None, None] for q in v)
+        t = (t - m) * r
+        t = torch.where(t >= 0, t, a * t)
+    wd = torch.from_numpy(w).double()
+    y = F.conv2d(t, wd, torch.from_numpy(b).double(), padding=pad)
+    size = F.conv2d(t.abs(), wd.abs(), torch.from_numpy(b).double().abs(), padding=pad)
+    return (y.relu() if act else y).numpy(), size.numpy()
+
+
+@pytest.mark.parametrize("c", CASES, ids=[str(c) for c in CASES])
+def test_edges(c, dev, ic):
+    print(f"[conv split] {c}", flush=True)
+    x, w, b, v = tensors(c, sum(c))
+    got = run(dev, ic, c, x, w, b, v)
+    ref, size = want(c, x, w, b, v)
+    worst = np.max(np.abs(got - ref) / (U * (25 * c[1] / 8 + 19) * size))
+    print(f"[conv split] worst {worst:.3f} of the bound", flush=True)
+    assert worst <= 1
+
+
+def test_values_that_are_not_finite(dev, ic):
+    c = (1, 18, 40, 160, 165, 2, 0, 0)
+    x, w, b, _ = tensors(c, 5)
+    x[0, 3, 0, 0] = np.inf
+    x[0, 17, 80, 70] = np.nan
+    x[0, 0, 159, 164] = 3.4e38  # above the largest bf16
+    w[7, 3, 2, 2] = 0           # inf * 0
+    w[:, 0] *= 0.5              # no output overflows
+    got = run(dev, ic, c, x, w, b, None)
+    ref, _ = want(c, x, w, b, None)
+    with np.errstate(over="ignore"):
+        ref = ref.astype(np.float32)
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)])
+    fine = np.isfinite(ref)
+    size = np.maximum(np.abs(ref[fine]), 4)
+    assert np.max(np.abs(got[fine] - ref[fine]) / size) <= 1e-5
