@@ -1,6 +1,6 @@
 /* SPDX-License-Identifier: Unlicense */
 
-/* Blockwise scaled dot-product attention on the fp32 matrix cores:
+/* Blockwise scaled dot-product attention on the matrix cores:
  * O = softmax(scale Q K^T) V per head, never storing the scores. The
  * contract is the reference's attention kernel (ops.cl:604-687,
  * ops.c:444-474 of i.coregistration.opencl): token-major operands with
@@ -10,7 +10,10 @@
  * A block holds 4 waves of 32 queries each (128 queries of one head)
  * and streams its range of keys in tiles of 32 through double-buffered
  * LDS, shared by the 4 waves, one barrier per tile; with 16-byte
- * aligned rows the next tile is read into registers a tile ahead:
+ * aligned rows the next tile is read into registers a tile ahead (the
+ * fp32 block, att_block_f32; attention_split_kernel does the same on the
+ * bf16 instructions, without loss, and is what 1 .. 64 and 97 .. 128
+ * channels a head run on):
  *  - the scores are computed transposed, S^T = K Q^T, with
  *    v_mfma_f32_32x32x2f32 (A = K from LDS, B = the wave's queries,
  *    pre-scaled and held in registers for the whole kernel), so that
@@ -38,6 +41,7 @@
 
 #include "common.h"
 #include "ops.h"
+#include "split.h"
 
 using namespace icoreg;
 
@@ -119,6 +123,19 @@ __device__ __forceinline__ void att_stash_direct(const float *K, int ldk,
     }
 }
 
+/* Arguments of the attention kernels (one image's operands; images bq .. bo
+ * floats apart). */
+struct att_args {
+    const float *Q, *K, *V;
+    float *O;
+    const unsigned char *kmask;
+    float *part_o;
+    float2 *part_ml;
+    int ldq, ldk, ldv, ldo, Nq, Nk, d, nh, tiles_per_split;
+    float scale;
+    long long bq, bk, bv, bo;
+};
+
 /* One block: 128 queries (4 waves x 32) of one head against the key
  * tiles [t0, t1) of 32 keys. K and V tiles are double-buffered in LDS
  * and shared by the 4 waves: the next tile (fetched into registers one
@@ -129,31 +146,32 @@ __device__ __forceinline__ void att_stash_direct(const float *K, int ldk,
  * one split the normalised output goes to O directly. MASK: a key mask
  * is given. */
 template <int ND, bool VEC, bool MASK>
-__global__ void __launch_bounds__(64 * ATT_NW)
-    attention_kernel(const float *__restrict__ Q, int ldq,
-                     const float *__restrict__ K, int ldk,
-                     const float *__restrict__ V, int ldv,
-                     float *__restrict__ O, int ldo, int Nq, int Nk, int d,
-                     float scale, const unsigned char *__restrict__ kmask,
-                     int tiles_per_split, float *__restrict__ part_o,
-                     float2 *__restrict__ part_ml, int nh, long long bq,
-                     long long bk, long long bv, long long bo)
+__device__ __forceinline__ void att_block_f32(const att_args &a, float *lds, int bx, int by,
+                                              int bz, int ny)
 {
+    const float *__restrict__ Q = a.Q, *__restrict__ K = a.K, *__restrict__ V = a.V;
+    float *__restrict__ O = a.O, *__restrict__ part_o = a.part_o;
+    float2 *__restrict__ part_ml = a.part_ml;
+    const unsigned char *__restrict__ kmask = a.kmask;
+    const int ldq = a.ldq, ldk = a.ldk, ldv = a.ldv, ldo = a.ldo;
+    const int Nq = a.Nq, Nk = a.Nk, d = a.d, nh = a.nh, tiles_per_split = a.tiles_per_split;
+    const float scale = a.scale;
+    const long long bq = a.bq, bk = a.bk, bv = a.bv, bo = a.bo;
     constexpr int DP = 32 * ND;     /* padded head dimension */
     constexpr int KP = DP + 1;      /* K tile row pitch (odd: no conflicts) */
     constexpr int VP = DP + 4;      /* V tile row pitch */
     constexpr int NS = DP / 2;      /* score MFMA steps */
     constexpr int NL = VEC ? ATT_KT * DP / 4 / (64 * ATT_NW)
                            : ATT_KT * DP / (64 * ATT_NW); /* loads / thread */
-    __shared__ __align__(16) float Ks[2][ATT_KT * KP];
-    __shared__ __align__(16) float Vs[2][ATT_KT * VP];
+    /* K tiles, then V tiles (16-byte rows). */
+    float *const Vs_ = lds, *const Ks_ = lds + 2 * ATT_KT * VP;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int h = blockIdx.y % nh, bi = blockIdx.y / nh;
+    const int h = by % nh, bi = by / nh;
     const int half = lane >> 5, col = lane & 31;
-    const int qi = (blockIdx.x * ATT_NW + wave) * 32 + col;
+    const int qi = (bx * ATT_NW + wave) * 32 + col;
     const int ntiles = (Nk + ATT_KT - 1) / ATT_KT;
-    const int t0 = blockIdx.z * tiles_per_split;
+    const int t0 = bz * tiles_per_split;
     const int t1 = min(ntiles, t0 + tiles_per_split);
     float q[NS];
     floatx16 o[ND];
@@ -185,20 +203,20 @@ __global__ void __launch_bounds__(64 * ATT_NW)
         if constexpr (VEC) {
             att_fetch<NL, DP>(kr4, vr4, K, ldk, V, ldv, t0 * ATT_KT, Nk, d,
                               tid);
-            att_stash<NL, DP, KP, VP>(kr4, vr4, Ks[0], Vs[0], tid);
+            att_stash<NL, DP, KP, VP>(kr4, vr4, Ks_, Vs_, tid);
             if (t0 + 1 < t1)
                 att_fetch<NL, DP>(kr4, vr4, K, ldk, V, ldv,
                                   (t0 + 1) * ATT_KT, Nk, d, tid);
         }
         else {
             att_stash_direct<NL, DP, KP, VP>(K, ldk, V, ldv, t0 * ATT_KT, Nk,
-                                             d, Ks[0], Vs[0], tid);
+                                             d, Ks_, Vs_, tid);
         }
     }
     __syncthreads();
     for (int t = t0; t < t1; t++) {
         const int k0 = t * ATT_KT, cur = (t - t0) & 1;
-        const float *ks = Ks[cur], *vs = Vs[cur];
+        const float *ks = Ks_ + cur * (ATT_KT * KP), *vs = Vs_ + cur * (ATT_KT * VP);
         floatx16 s;
 
 #pragma unroll
@@ -296,8 +314,8 @@ __global__ void __launch_bounds__(64 * ATT_NW)
          * before the previous barrier), then its successor's loads. */
         if (t + 1 < t1) {
             if constexpr (VEC) {
-                att_stash<NL, DP, KP, VP>(kr4, vr4, Ks[cur ^ 1], Vs[cur ^ 1],
-                                          tid);
+                att_stash<NL, DP, KP, VP>(kr4, vr4, Ks_ + (cur ^ 1) * (ATT_KT * KP),
+                                          Vs_ + (cur ^ 1) * (ATT_KT * VP), tid);
                 if (t + 2 < t1)
                     att_fetch<NL, DP>(kr4, vr4, K, ldk, V, ldv,
                                       (t + 2) * ATT_KT, Nk, d, tid);
@@ -305,8 +323,8 @@ __global__ void __launch_bounds__(64 * ATT_NW)
             else {
                 att_stash_direct<NL, DP, KP, VP>(K, ldk, V, ldv,
                                                  (t + 1) * ATT_KT, Nk, d,
-                                                 Ks[cur ^ 1], Vs[cur ^ 1],
-                                                 tid);
+                                                 Ks_ + (cur ^ 1) * (ATT_KT * KP),
+                                                 Vs_ + (cur ^ 1) * (ATT_KT * VP), tid);
             }
         }
 
@@ -357,7 +375,7 @@ __global__ void __launch_bounds__(64 * ATT_NW)
     }
     else {
         const long long row =
-            ((long long)blockIdx.z * gridDim.y + blockIdx.y) * Nq + qi;
+            ((long long)bz * ny + by) * Nq + qi;
         float *out = part_o + row * DP;
 
 #pragma unroll
@@ -367,6 +385,340 @@ __global__ void __launch_bounds__(64 * ATT_NW)
                 out[tt * 32 + (r >> 2) * 8 + half * 4 + (r & 3)] = o[tt][r];
         if (half == 0)
             part_ml[row] = make_float2(m, l);
+    }
+}
+
+/* Floats of LDS of att_block_f32: both operands' double-buffered tiles. */
+template <int ND> constexpr int att_f32_lds = 2 * ATT_KT * (2 * 32 * ND + 5);
+
+/* The block on the fp32 instructions (65 .. 96 channels a head). */
+template <int ND, bool VEC, bool MASK>
+__global__ void __launch_bounds__(64 * ATT_NW) attention_kernel(const att_args a)
+{
+    __shared__ __align__(16) float lds[att_f32_lds<ND>];
+
+    att_block_f32<ND, VEC, MASK>(a, lds, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.y);
+}
+
+/* The same block on the bf16 instructions: queries, keys, values and
+ * probabilities split exactly into three bf16 parts, six products each
+ * (split.h). K tiles lie in LDS as [part][key][channels] and V tiles
+ * transposed, [part][channel][keys], the keys of a row in the order in which
+ * the score product leaves them in the lanes: slot j of lane half h of step u
+ * is key 16 u + 8 (j / 4) + 4 h + j % 4, so the split probabilities are the
+ * second product's operands as they stand. 16-byte chunks are stored XORed
+ * with row bits, 16 rows to 64 banks. A score's 5 small products per 16
+ * channels are summed before the large ones.
+ *
+ * Per 32 keys, 32 queries and 64 channels 48 products (1536 cycles) run
+ * beside 16 exponentials and 32 splits a lane (about 1200 cycles of vector
+ * instructions): bound by those, by the loads' latency and by the two units
+ * overlapping only between the 3 blocks that the registers hold. Measured on
+ * an MI355X with the merge, against the fp32 block: 2 x 16 heads of 64, 1601
+ * tokens 223 -> 147 us (143 TFLOP/s); 16 heads of 64, 785 tokens 56 -> 40;
+ * 2 x 8 heads of 32, 400 tokens 18.7 -> 16; 2 x 16 heads of 32, 1601 tokens
+ * 138 -> 88; 8 heads of 128, 1600 tokens 167 -> 95; 2 x 16 heads of 128, 2304
+ * tokens 937 -> 595; 4 heads of 64, 49 tokens 12.2 -> 11.2. Tried: the next
+ * tile's scores beside this one's softmax in one wave, 2 blocks a CU (64
+ * channels 147 -> 155, 128 channels 596 -> 604). Error against 64 bits half
+ * of the fp32 block's (4.1e-7, 8.4e-7: its 64 terms round each time). The
+ * order of the blocks gave 188 -> 174 of those 147, loads without a range
+ * check per value (rows past the keys read the last key again) the rest.
+ * 65 .. 96 channels stay on the fp32 block: rows of 12 chunks would not
+ * spread over the banks this way.
+ *
+ * If a sum is not finite (an infinity or NaN among the operands has no
+ * split), the block runs again on the fp32 instructions. */
+template <int ND, bool VEC, bool MASK>
+__global__ void __launch_bounds__(64 * ATT_NW, ND == 4 ? 1 : 3)
+    attention_split_kernel(const att_args a)
+{
+    constexpr int DP = 32 * ND, CH = DP / 8;  /* chunks of a K row */
+    constexpr int RW = 16 / CH < 1 ? 1 : 16 / CH; /* K rows in 256 bytes */
+    constexpr int PK = ATT_KT * CH;           /* chunks of a part: K and V alike */
+    constexpr int NT = 64 * ATT_NW, NL = (PK + NT - 1) / NT;
+    constexpr int LDSF = 2 * 6 * PK * 4;
+    __shared__ split_u4 lds[(LDSF > att_f32_lds<ND> ? LDSF : att_f32_lds<ND>) / 4 + 1];
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    /* Blocks are dealt to the 8 XCDs in turn: XCD x takes the x-th band of
+     * the order (image and head, key range, queries), so that a head's K and
+     * V stay in one L2. */
+    const int nx = gridDim.x, ny = gridDim.y, T = nx * ny * gridDim.z;
+    const int id = (blockIdx.z * ny + blockIdx.y) * nx + blockIdx.x;
+    const int unit = (id & 7) * (T >> 3) + min(id & 7, T & 7) + (id >> 3);
+    const int bx = unit % nx, bz = unit / nx % gridDim.z;
+    const int by = unit / (nx * gridDim.z), h = by % a.nh, bi = by / a.nh;
+    const int half = lane >> 5, col = lane & 31, d = a.d, Nk = a.Nk;
+    const int qi = (bx * ATT_NW + wave) * 32 + col;
+    const int ntiles = (Nk + ATT_KT - 1) / ATT_KT;
+    const int t0 = bz * a.tiles_per_split, t1 = min(ntiles, t0 + a.tiles_per_split);
+    const float *Q = a.Q + bi * a.bq + (long long)h * d;
+    const float *K = a.K + bi * a.bk + (long long)h * d;
+    const float *V = a.V + bi * a.bv + (long long)h * d;
+    /* Threads past the chunks (32 channels a head): none in K, all in V. */
+    constexpr bool APART = PK < NT;
+    const bool has_k = !APART || tid < PK;
+    const int vt = APART ? tid - PK : tid;
+    float kr[NL][8], vr[NL][8];
+    split_u4 q[2 * ND][3];
+    floatx16 o[ND];
+    float m = -INFINITY, l = 0.0f;
+
+#pragma unroll
+    for (int st = 0; st < 2 * ND; st++) {
+        float x[8];
+
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int dd = st * 16 + half * 8 + j;
+
+            x[j] = qi < a.Nq && dd < d
+                       ? Q[(long long)qi * a.ldq + dd] * (a.scale * 1.4426950408889634f)
+                       : 0.0f;
+        }
+        split8(x, q[st][0], q[st][1], q[st][2]);
+    }
+#pragma unroll
+    for (int t = 0; t < ND; t++)
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+            o[t][r] = 0.0f;
+
+    /* Tile k0 into registers: K chunk e is key e / CH, channels 8 (e % CH)
+     * ..; V chunk e channel e % DP, slots 8 (e / DP) .. + 7 (keys that a
+     * wave's lanes share). Past Nk and d the last key and the last channels
+     * are read again: the queries' channels there are 0, such keys get no
+     * probability and such output channels are not stored. */
+    auto fetch = [&](int k0) {
+        const float *kt = K + (long long)k0 * a.ldk;
+        const int last = Nk - 1 - k0;
+
+        if (has_k) {
+#pragma unroll
+            for (int i = 0; i < NL; i++) {
+                const int e = tid + NT * i, dd = e % CH * 8;
+                const float *p = kt + (long long)min(e / CH, last) * a.ldk;
+
+                if (VEC) {
+                    const float4 x = *(const float4 *)(p + min(dd, d - 4));
+                    const float4 y = *(const float4 *)(p + min(dd + 4, d - 4));
+
+                    kr[i][0] = x.x, kr[i][1] = x.y, kr[i][2] = x.z, kr[i][3] = x.w;
+                    kr[i][4] = y.x, kr[i][5] = y.y, kr[i][6] = y.z, kr[i][7] = y.w;
+                }
+                else {
+#pragma unroll
+                    for (int j = 0; j < 8; j++)
+                        kr[i][j] = p[min(dd + j, d - 1)];
+                }
+            }
+        }
+        if (!APART || !has_k) {
+#pragma unroll
+            for (int i = 0; i < NL; i++) {
+                const int e = vt + NT * i;
+                const unsigned dd = min(e % DP, d - 1);
+                const int c = ND == 1 ? e / DP : __builtin_amdgcn_readfirstlane(e / DP);
+
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const int kk = (c >> 1) * 16 + (j >> 2) * 8 + (c & 1) * 4 + (j & 3);
+
+                    vr[i][j] = (V + (long long)(k0 + min(kk, last)) * a.ldv)[dd];
+                }
+            }
+        }
+    };
+    auto stash = [&](split_u4 *ks) {
+        split_u4 *vs = ks + 3 * PK, x, y, z;
+
+        if (has_k) {
+#pragma unroll
+            for (int i = 0; i < NL; i++) {
+                const int e = tid + NT * i, key = e / CH;
+                const int at = key * CH + ((e % CH) ^ (key / RW % CH));
+
+                split8(kr[i], x, y, z);
+                ks[at] = x;
+                ks[PK + at] = y;
+                ks[2 * PK + at] = z;
+            }
+        }
+        if (!APART || !has_k) {
+#pragma unroll
+            for (int i = 0; i < NL; i++) {
+                const int e = vt + NT * i, dd = e % DP;
+                const int at = dd * 4 + ((e / DP) ^ (dd >> 2 & 3));
+
+                split8(vr[i], x, y, z);
+                vs[at] = x;
+                vs[PK + at] = y;
+                vs[2 * PK + at] = z;
+            }
+        }
+    };
+    constexpr int pa[6] = {0, 2, 1, 0, 1, 0}, pb[6] = {2, 0, 1, 1, 0, 0};
+
+    if (t0 < t1) {
+        fetch(t0 * ATT_KT);
+        stash(lds);
+        if (t0 + 1 < t1)
+            fetch((t0 + 1) * ATT_KT);
+    }
+    __syncthreads();
+    for (int t = t0; t < t1; t++) {
+        const int k0 = t * ATT_KT, cur = (t - t0) & 1;
+        const split_u4 *ks = lds + cur * (6 * PK), *vs = ks + 3 * PK;
+        auto key = [&](int p, int st) {
+            return __builtin_bit_cast(
+                split_b8, ks[p * PK + col * CH + ((2 * st + half) ^ (col / RW % CH))]);
+        };
+        floatx16 s;
+
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+            s[r] = 0.0f;
+#pragma unroll
+        for (int st = 0; st < 2 * ND; st++) {
+            const split_b8 kf[3] = {key(0, st), key(1, st), key(2, st)};
+
+#pragma unroll
+            for (int w = 0; w < 5; w++)
+                s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                    kf[pa[w]], __builtin_bit_cast(split_b8, q[st][pb[w]]), s, 0, 0, 0);
+        }
+#pragma unroll
+        for (int st = 0; st < 2 * ND; st++)
+            s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                key(0, st), __builtin_bit_cast(split_b8, q[st][0]), s, 0, 0, 0);
+
+        /* Online softmax as in att_block_f32. */
+        float p[16], mx = -INFINITY, sum = 0.0f;
+
+        if (MASK || k0 + ATT_KT > Nk) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int kk = k0 + (r >> 2) * 8 + half * 4 + (r & 3);
+                bool keep = kk < Nk;
+
+                if (MASK)
+                    keep = keep && a.kmask[min(kk, Nk - 1)] != 0;
+                p[r] = keep ? s[r] : -INFINITY;
+                mx = fmaxf(mx, p[r]);
+            }
+        }
+        else {
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                p[r] = s[r];
+                mx = fmaxf(mx, p[r]);
+            }
+        }
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const bool need = mx > m + ATT_TAU;
+
+        if (__any(need)) {
+            const float mn = need ? mx : m;
+            const float corr =
+                need ? (m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mn)) : 1.0f;
+
+            m = mn;
+            l *= corr;
+#pragma unroll
+            for (int tt = 0; tt < ND; tt++)
+#pragma unroll
+                for (int r = 0; r < 16; r++)
+                    o[tt][r] *= corr;
+        }
+        {
+            /* No key kept yet: every score is -infinity, 2^-infinity = 0. */
+            const float ref = m == -INFINITY ? 0.0f : m;
+
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                p[r] = __builtin_amdgcn_exp2f(p[r] - ref);
+                sum += p[r];
+            }
+        }
+        l += sum + __shfl_xor(sum, 32, 64);
+
+        /* The next tile into the other buffer (last read one tile ago,
+         * before the previous barrier), then its successor's loads. */
+        if (t + 1 < t1) {
+            stash(lds + (cur ^ 1) * (6 * PK));
+            if (t + 2 < t1)
+                fetch((t + 2) * ATT_KT);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            float x[8];
+            split_u4 pp[3];
+
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+                x[j] = p[8 * u + j];
+            split8(x, pp[0], pp[1], pp[2]);
+#pragma unroll
+            for (int tt = 0; tt < ND; tt++) {
+                const int dd = tt * 32 + col;
+                split_b8 vf[3];
+
+#pragma unroll
+                for (int k = 0; k < 3; k++)
+                    vf[k] = __builtin_bit_cast(
+                        split_b8, vs[k * PK + dd * 4 + ((2 * u + half) ^ (dd >> 2 & 3))]);
+#pragma unroll
+                for (int w = 0; w < 6; w++)
+                    o[tt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                        vf[pa[w]], __builtin_bit_cast(split_b8, pp[pb[w]]), o[tt], 0, 0, 0);
+            }
+        }
+        __syncthreads();
+    }
+
+    {
+        float z = l * 0.0f;
+
+#pragma unroll
+        for (int tt = 0; tt < ND; tt++)
+#pragma unroll
+            for (int r = 0; r < 16; r++)
+                z = fmaf(o[tt][r], 0.0f, z);
+        if (__syncthreads_or(z != 0.0f)) {
+            att_block_f32<ND, false, MASK>(a, (float *)lds, bx, by, bz, ny);
+            return;
+        }
+    }
+    if (qi >= a.Nq)
+        return;
+    if (!a.part_o) {
+        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+        float *out = a.O + bi * a.bo + (long long)qi * a.ldo + (long long)h * d;
+
+#pragma unroll
+        for (int tt = 0; tt < ND; tt++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int dd = tt * 32 + (r >> 2) * 8 + half * 4 + (r & 3);
+
+                if (dd < d)
+                    out[dd] = l > 0.0f ? o[tt][r] * inv : 0.0f;
+            }
+    }
+    else {
+        const long long row = ((long long)bz * ny + by) * a.Nq + qi;
+        float *out = a.part_o + row * DP;
+
+#pragma unroll
+        for (int tt = 0; tt < ND; tt++)
+#pragma unroll
+            for (int g = 0; g < 4; g++)
+                *(float4 *)(out + tt * 32 + g * 8 + half * 4) =
+                    make_float4(o[tt][4 * g], o[tt][4 * g + 1], o[tt][4 * g + 2],
+                                o[tt][4 * g + 3]);
+        if (half == 0)
+            a.part_ml[row] = make_float2(m, l);
     }
 }
 
@@ -452,6 +804,43 @@ __global__ void __launch_bounds__(256)
                  : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 }
 
+/* Key ranges of attention_split_kernel, at most `most`: the fewest
+ * microseconds of the slowest CU (its share of the blocks, each a range's
+ * tiles and about one for its start) and of the merge (3, and merge_us for
+ * the partials of each range, written and read). A tile of one block takes
+ * about 0.6 + 0.75 ND, a block beside it 0.55 more, as many as the
+ * registers hold (4, 3, 1). Against the fp32 kernel's count (`most`, two
+ * blocks per CU and evened out), which cuts finer than one block a CU
+ * wherever few heads leave the chip short: 1600 tokens, 8 heads of 128, 2
+ * ranges instead of 5 121 -> 95 us; 785 x 16 x 64, 2 instead of 5 43.5 -> 37;
+ * 2 x 676 x 8 x 32, 2 instead of 7 27.9 -> 22.7; 2 x 1601 x 16 x 64 keeps
+ * its 3 (147; 1: 152, 2: 164). */
+template <int ND>
+static int split_count(int most, long long blocks, int ntiles, int cus, double merge_us,
+                       int &tps)
+{
+    constexpr int held = ND == 1 ? 4 : ND == 2 ? 3 : 1;
+    double best = 0;
+    int n = most;
+
+    for (int s = 1; s <= most; s++) {
+        const int len = (ntiles + s - 1) / s;
+        const int ranges = len > 0 ? (ntiles + len - 1) / len : 1;
+        const long long each = (blocks * ranges + cus - 1) / cus;
+        const double rounds = (double)(each / held) * (0.45 + 0.55 * held) +
+                              (each % held ? 0.45 + 0.55 * (each % held) : 0.0);
+        const double us =
+            (len + 1) * rounds * (0.6 + 0.75 * ND) + (ranges > 1 ? 3 + ranges * merge_us : 0.0);
+
+        if (s == 1 || us < best) {
+            best = us;
+            n = ranges;
+            tps = len;
+        }
+    }
+    return n;
+}
+
 /* Partials of the key splits: the ops work buffer (grown on demand), or,
  * for ops_attention_noalloc, the fixed device array `fixed` of
  * fixed_bytes bytes (too small a one is a fatal error). */
@@ -494,37 +883,46 @@ static void launch_nd(struct ops *ops, hipStream_t st, int nb, int nh,
     }
     tps = ntiles > 0 ? (ntiles + nsplit - 1) / nsplit : 0;
     nsplit = tps > 0 ? (ntiles + tps - 1) / tps : 1;
+    /* What the scratch must hold: the most splits that are considered. */
+    const size_t rows = (size_t)nsplit * nb * nh * Nq;
+    const size_t ob = nsplit > 1 ? rows * 32 * ND * sizeof(float) : 0;
+
+    if (nsplit > 1 && fixed && ob + rows * sizeof(float2) > fixed_bytes)
+        icoreg_fatal("ops_attention_noalloc: the key-split partials (%zu bytes) "
+                     "exceed the %zu-byte scratch array",
+                     ob + rows * sizeof(float2), fixed_bytes);
+    if (ND != 3)
+        nsplit = split_count<ND>(nsplit, (long long)qb * nh * nb, ntiles,
+                                 ops->ocl->cu_count > 0 ? ops->ocl->cu_count : 256,
+                                 5e-7 * 4 * nb * nh * Nq * 32 * ND, tps);
+
+    auto launch = [&](dim3 grid, float *po, float2 *pml) {
+        const att_args a = {Q,  K,  V, O,  kmask, po,    pml, ldq, ldk, ldv, ldo,
+                            Nq, Nk, d, nh, tps,   scale, bq,  bk,  bv,  bo};
+
+        if constexpr (ND == 3)
+            hipLaunchKernelGGL((attention_kernel<ND, VEC, MASK>), grid, dim3(64 * ATT_NW), 0, st,
+                               a);
+        else
+            hipLaunchKernelGGL((attention_split_kernel<ND, VEC, MASK>),
+                               grid, dim3(64 * ATT_NW), 0, st, a);
+    };
+
     if (nsplit == 1) {
-        hipLaunchKernelGGL((attention_kernel<ND, VEC, MASK>),
-                           dim3((unsigned)qb, (unsigned)(nh * nb), 1),
-                           dim3(64 * ATT_NW), 0, st, Q, ldq, K, ldk, V, ldv,
-                           O, ldo, Nq, Nk, d, scale, kmask, tps, nullptr,
-                           nullptr, nh, bq, bk, bv, bo);
+        launch(dim3((unsigned)qb, (unsigned)(nh * nb), 1), nullptr, nullptr);
         return;
     }
     {
-        const size_t rows = (size_t)nsplit * nb * nh * Nq;
-        const size_t ob = rows * 32 * ND * sizeof(float);
         float *po;
 
-        if (fixed) {
-            if (ob + rows * sizeof(float2) > fixed_bytes)
-                icoreg_fatal("ops_attention_noalloc: the key-split partials (%zu bytes) "
-                             "exceed the %zu-byte scratch array",
-                             ob + rows * sizeof(float2), fixed_bytes);
+        if (fixed)
             po = fixed;
-        }
         else
             po = (float *)scratch_get(ops, ob + rows * sizeof(float2))->ptr;
         float2 *pml = (float2 *)((char *)po + ob);
         const long long total = (long long)nb * Nq * nh * d;
 
-        hipLaunchKernelGGL((attention_kernel<ND, VEC, MASK>),
-                           dim3((unsigned)qb, (unsigned)(nh * nb),
-                                (unsigned)nsplit),
-                           dim3(64 * ATT_NW), 0, st, Q, ldq, K, ldk, V, ldv,
-                           O, ldo, Nq, Nk, d, scale, kmask, tps, po, pml, nh,
-                           bq, bk, bv, bo);
+        launch(dim3((unsigned)qb, (unsigned)(nh * nb), (unsigned)nsplit), po, pml);
         if (d % 4 == 0 && ldo % 4 == 0 && bo % 4 == 0 && ((uintptr_t)O & 15) == 0)
             hipLaunchKernelGGL(attn_merge4_kernel,
                                dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0,

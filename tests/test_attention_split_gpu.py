@@ -1,0 +1,115 @@
+# SPDX-License-Identifier: Unlicense
+"""GPU: attention on the bf16 matrix instructions against float64 softmax
+attention, at the edges of its tiles, key ranges and loads.
+
+Bound: a score's six kept bf16 products lose at most U (d / 8 + 16) of
+scale sum |q k| (U = 2^-24: d / 8 additions, the groups' alignment, the
+products left out) and the query's scaling 2 U more, so a probability is off
+by that much relatively, and by 4 U for its exponential; the numerator and
+the denominator both carry it. The sum over the keys adds U (Nk / 8 + 16),
+the merge of key ranges and the division 32 U at most, of sum p |v|."""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+U = 2.0 ** -24
+
+# (images, Nq, Nk, heads, d, float offset of the operands, mask)
+SHAPES = [
+    # One of everything; no channel, key or query tile full.
+    (1, 1, 1, 1, 1, 0, 0),
+    (1, 33, 31, 3, 5, 0, 1),
+    # 32 channels a head, and one to either side; 16-byte loads and not.
+    (1, 129, 33, 8, 32, 0, 0),
+    (2, 128, 64, 2, 31, 0, 0),
+    (1, 127, 65, 2, 33, 0, 1),
+    (1, 31, 95, 4, 36, 0, 0),
+    (1, 65, 97, 4, 64, 1, 0),
+    (2, 400, 400, 8, 32, 0, 0),
+    # Key ranges, the last one shorter; few queries over many keys.
+    (1, 100, 1000, 8, 64, 0, 1),
+    (2, 785, 785, 4, 64, 0, 0),
+    # 97 .. 128 channels.
+    (1, 40, 130, 2, 97, 0, 0),
+    (1, 129, 63, 2, 100, 0, 1),
+    (1, 300, 333, 4, 128, 0, 0),
+    # No key at all: zeros.
+    (1, 40, 0, 2, 64, 0, 0),
+]
+
+
+def run(dev, ic, q, k, v, scale, off=0, mask=None):
+    nb, Nq, nh, d = q.shape
+    Nk, ld = k.shape[1], nh * d
+
+    def up(x):
+        return dev.upload(np.concatenate([np.zeros(off, np.float32), x.ravel(),
+                                          np.zeros(4, np.float32)]))
+
+    Q, K, V = up(q), up(k), up(v)
+    O = dev.upload(np.full(nb * Nq * ld, 7.0, np.float32))
+    keep = dev.upload(mask) if mask is not None else None
+    dev.api.ops_attention_batch(dev.po, nb, ic.mat(Q, off, ld), Nq * ld, ic.mat(K, off, ld),
+                                Nk * ld, ic.mat(V, off, ld), Nk * ld, ic.mat(O, 0, ld), Nq * ld,
+                                Nq, Nk, nh, d, scale, ic.mem(keep) if keep is not None else None)
+    return dev.read(O, nb * Nq * ld).reshape(nb, Nq, nh, d)
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=[str(s) for s in SHAPES])
+def test_edges(shape, dev, ic):
+    nb, Nq, Nk, nh, d, off, masked = shape
+    print(f"[attention split] {shape}", flush=True)
+    rng = np.random.default_rng(Nq + 3 * Nk + d)
+    q = rng.standard_normal((nb, Nq, nh, d)).astype(np.float32)
+    k = rng.standard_normal((nb, Nk, nh, d)).astype(np.float32)
+    v = rng.standard_normal((nb, Nk, nh, d)).astype(np.float32)
+    mask = (rng.random(Nk) < 0.7).astype(np.uint8) if masked else None
+    scale = float(np.float32(1.5 / np.sqrt(d)))
+    got = run(dev, ic, q, k, v, scale, off, mask)
+    if Nk == 0:
+        assert not got.any()
+        return
+    qh, kh, vh = (x.astype(np.float64).transpose(0, 2, 1, 3) for x in (q, k, v))
+    s = scale * qh @ kh.swapaxes(2, 3)
+    size = scale * np.abs(qh) @ np.abs(kh).swapaxes(2, 3)
+    if masked:
+        s[..., mask == 0] = -np.inf
+        size[..., mask == 0] = 0
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    want = (p @ vh).transpose(0, 2, 1, 3)
+    rel = 2 * ((d / 8 + 18) * size.max(-1) + 4) + Nk / 8 + 48
+    bound = U * (rel[..., None] * (p @ np.abs(vh))).transpose(0, 2, 1, 3)
+    worst = np.max(np.abs(got - want) / bound)
+    print(f"[attention split] worst {worst:.3f} of the bound", flush=True)
+    assert worst <= 1
+
+
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_values_that_are_not_finite(d, dev, ic):
+    """Infinities, NaN and values above the largest bf16 give what the fp32
+    instructions give (a query whose sum of probabilities is NaN gets zeros,
+    as one with no key left does); the other heads keep their values."""
+    rng = np.random.default_rng(d)
+    nh, Nq, Nk = 4, 70, 90
+    q, k, v = (rng.standard_normal((1, n, nh, d)).astype(np.float32) for n in (Nq, Nk, Nk))
+    scale = float(1.0 / np.sqrt(d))
+    clean = run(dev, ic, q, k, v, scale)
+    v[0, 88, 0, 3] = np.inf
+    v[0, 5, 0, 7] = 3.4e38
+    k[0, 40, 1, 0] = np.nan
+    q[0, 9, 2, 1] = np.inf
+    got = run(dev, ic, q, k, v, scale)[0]
+    qh, kh = q[0, :, 0].astype(np.float64), k[0, :, 0].astype(np.float64)
+    p = np.exp(scale * qh @ kh.T)
+    p /= p.sum(-1, keepdims=True)
+    assert np.all(got[:, 0, 3] == np.inf)
+    assert np.allclose(got[:, 0, 7], p[:, 5] * 3.4e38, rtol=1e-4)
+    assert np.allclose(np.delete(got[:, 0], [3, 7], 1), np.delete(clean[0, :, 0], [3, 7], 1),
+                       rtol=0, atol=1e-4)
+    assert not got[:, 1].any() and not got[9, 2].any()
+    rows = np.delete(np.arange(Nq), 9)
+    assert np.allclose(got[rows, 2], clean[0, rows, 2], rtol=0, atol=1e-4)
+    assert np.array_equal(got[:, 3], clean[0, :, 3])
