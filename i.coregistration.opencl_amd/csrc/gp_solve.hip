@@ -29,10 +29,11 @@
  * Synchronisation, inside the kernels: the diagonal kernel of block b
  * sets a flag once its factor and inverse are stored, which panel b's
  * first products on the second stream poll before reading them; and it
- * waits itself for a flag that a one-wave kernel sets on the second
- * stream after panel b - 2's trailing update. Neither stream then holds
+ * waits itself for a flag that panel b - 1's first launch on the second
+ * stream sets as it starts, after panel b - 2's trailing update. Neither stream then holds
  * a stream wait or an event record between its kernels (each costs 5-7
- * us of command-processor time, on the solve's critical path). Every
+ * us of command-processor time, on the solve's critical path, and so did a
+ * kernel of its own for the flag). Every
  * wait is bounded; one that gives up sets info = -1 and its kernel ends
  * (the caller then runs the solve again with event waits). Under stream
  * capture (a graph has no order between branches that an in-kernel wait
@@ -53,21 +54,25 @@
 
 using namespace icoreg;
 
+typedef double gp_d4 __attribute__((ext_vector_type(4)));
+
 #define GP_NB 64 /* panel width */
+#define GP_SB 16 /* columns factored between two updates of their block */
 #define DG_T 64  /* GEMM output tile */
 #define DG_K 32  /* GEMM reduction chunk */
 
 /* C = alpha A B + beta C with A(i, q) = A[i a_ri + q a_rk], B(q, j) =
  * B[q b_rk + j b_rj], C(i, j) = C[i c_ri + j]; lower: skip output tiles
- * strictly above the diagonal; skip00: leave output tile (0, 0) alone. */
+ * strictly above the diagonal; skip00: leave output tile (0, 0) alone.
+ * The matrices have less than 2^31 values: 32-bit indices. */
 struct dg_args {
     int M, N, K;
     const double *A;
-    long long a_ri, a_rk;
+    int a_ri, a_rk;
     const double *B;
-    long long b_rk, b_rj;
+    int b_rk, b_rj;
     double *C;
-    long long c_ri;
+    int c_ri;
     double alpha;
     int beta, lower;
     int skip00;
@@ -77,23 +82,35 @@ struct dg_args {
  * wait (when given): a flag the launch's blocks poll (one thread each,
  * device-coherent loads, at most spin_max polls, then an acquire) before
  * they read their operands; a wait that gives up sets *info = -1 and
- * goes on, so that the launch still ends. */
+ * goes on, so that the launch still ends. mark (when given): a flag set
+ * as the launch starts, which says that the launches before it on its
+ * stream have finished (device-coherent store). */
 #define DG_MAXP 3
 struct dg_set {
     dg_args p[DG_MAXP];
     const int *wait;
     int spin_max;
     int *info;
+    int *mark;
 };
 
-__global__ void __launch_bounds__(256) dgemm_kernel(dg_set pr)
+/* 64 x 64 outputs a block on v_mfma_f64_16x16x4f64, 32 x 32 a wave. The
+ * products are short (64 terms): bound by the round trips of C and of the
+ * two chunks, so registers for 3 blocks a CU and 32-bit indices count (64-bit
+ * ones took as long as the products). The solve at n = 1600, d = 512 with 4 x
+ * 4 outputs a thread on the vector unit 1073 us, so 967, with 3 blocks a CU
+ * and no flag kernel 890, with 32-bit indices 883 -> 814. */
+__global__ void __launch_bounds__(256, 3) dgemm_kernel(dg_set pr)
 {
     __shared__ double As[DG_K][DG_T + 1], Bs[DG_K][DG_T + 1];
     const dg_args &a = pr.p[blockIdx.z];
-    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
+    const int tid = threadIdx.x, wave = tid >> 6, kq = (tid & 63) >> 4, l16 = tid & 15;
     const int i0 = blockIdx.y * DG_T, j0 = blockIdx.x * DG_T;
-    double acc[4][4], cprev[4][4];
+    const int wi = 32 * (wave >> 1), wj = 32 * (wave & 1); /* the wave's 32 x 32 */
+    gp_d4 acc[2][2], cprev[2][2];
 
+    if (pr.mark && blockIdx.x + blockIdx.y + blockIdx.z == 0 && tid == 0)
+        __hip_atomic_store(pr.mark, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (i0 >= a.M || j0 >= a.N || (a.lower && j0 > i0 + DG_T - 1) ||
         (a.skip00 && i0 == 0 && j0 == 0))
         return;
@@ -113,18 +130,17 @@ __global__ void __launch_bounds__(256) dgemm_kernel(dg_set pr)
     /* The accumulated C is read at the start, so that its latency
      * overlaps the products. */
 #pragma unroll
-    for (int p = 0; p < 4; p++)
+    for (int p = 0; p < 2; p++)
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int i = min(i0 + ty + 16 * p, a.M - 1), j = min(j0 + tx + 16 * r, a.N - 1);
+        for (int r = 0; r < 2; r++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int i = min(i0 + wi + 16 * p + kq + 4 * v, a.M - 1);
+                const int j = min(j0 + wj + 16 * r + l16, a.N - 1);
 
-            cprev[p][r] = a.beta ? a.C[(long long)i * a.c_ri + j] : 0.0;
-        }
-#pragma unroll
-    for (int p = 0; p < 4; p++)
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-            acc[p][q] = 0.0;
+                cprev[p][r][v] = a.beta ? a.C[i * a.c_ri + j] : 0.0;
+                acc[p][r][v] = 0.0;
+            }
     /* 32 x 64 of A and of B per chunk, 8 values per thread, the
      * unit-stride index fastest across threads. Every load reads a valid
      * address (indices clamped to the last row / column) and the value is
@@ -145,10 +161,8 @@ __global__ void __launch_bounds__(256) dgemm_kernel(dg_set pr)
 
             oka[t] = i0 + i < a.M && k0 + q < a.K;
             okb[t] = j0 + j < a.N && k0 + qb < a.K;
-            va[t] = a.A[(long long)min(i0 + i, a.M - 1) * a.a_ri +
-                        (long long)min(k0 + q, a.K - 1) * a.a_rk];
-            vb[t] = a.B[(long long)min(k0 + qb, a.K - 1) * a.b_rk +
-                        (long long)min(j0 + j, a.N - 1) * a.b_rj];
+            va[t] = a.A[min(i0 + i, a.M - 1) * a.a_ri + min(k0 + q, a.K - 1) * a.a_rk];
+            vb[t] = a.B[min(k0 + qb, a.K - 1) * a.b_rk + min(j0 + j, a.N - 1) * a.b_rj];
         }
     };
     fetch(0);
@@ -167,37 +181,35 @@ __global__ void __launch_bounds__(256) dgemm_kernel(dg_set pr)
         __syncthreads();
         if (k0 + DG_K < a.K)
             fetch(k0 + DG_K);
-#pragma unroll 8
-        for (int q = 0; q < DG_K; q++) {
-            double av[4], bv[4];
+#pragma unroll
+        for (int q = 0; q < DG_K; q += 4) {
+            double av[2], bv[2];
 
 #pragma unroll
-            for (int p = 0; p < 4; p++) {
-                av[p] = As[q][ty + 16 * p];
-                bv[p] = Bs[q][tx + 16 * p];
+            for (int p = 0; p < 2; p++) {
+                av[p] = As[q + kq][wi + 16 * p + l16];
+                bv[p] = Bs[q + kq][wj + 16 * p + l16];
             }
 #pragma unroll
-            for (int p = 0; p < 4; p++)
+            for (int p = 0; p < 2; p++)
 #pragma unroll
-                for (int r = 0; r < 4; r++)
-                    acc[p][r] = fma(av[p], bv[r], acc[p][r]);
+                for (int r = 0; r < 2; r++)
+                    acc[p][r] =
+                        __builtin_amdgcn_mfma_f64_16x16x4f64(av[p], bv[r], acc[p][r], 0, 0, 0);
         }
         __syncthreads();
     }
 #pragma unroll
-    for (int p = 0; p < 4; p++) {
-        const int i = i0 + ty + 16 * p;
-
-        if (i >= a.M)
-            continue;
+    for (int p = 0; p < 2; p++)
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int j = j0 + tx + 16 * r;
+        for (int r = 0; r < 2; r++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int i = i0 + wi + 16 * p + kq + 4 * v, j = j0 + wj + 16 * r + l16;
 
-            if (j < a.N)
-                a.C[(long long)i * a.c_ri + j] = a.alpha * acc[p][r] + cprev[p][r];
-        }
-    }
+                if (i < a.M && j < a.N)
+                    a.C[i * a.c_ri + j] = a.alpha * acc[p][r][v] + cprev[p][r][v];
+            }
 }
 
 /* ---- the diagonal block ------------------------------------------------------------ */
@@ -225,8 +237,6 @@ __device__ __forceinline__ double readlane_d(double v, int l)
                     (unsigned)__builtin_amdgcn_readlane((int)b, l));
 }
 
-typedef double gp_d4 __attribute__((ext_vector_type(4)));
-
 /* Polls of a panel flag before the diagonal kernel gives up (with a
  * 64-clock sleep each: about 0.1 s, far beyond any trailing update): the wait
  * then ends with info = -1 instead of hanging. */
@@ -249,37 +259,33 @@ typedef double gp_d4 __attribute__((ext_vector_type(4)));
  *    A(l % 16, l / 16) and B(l / 16, l % 16) and holds D(l / 16 + 4 v,
  *    l % 16); the fp32 16 x 16 x 4 form holds rows 4 (l / 16) + v
  *    instead). Its operands (the block row of A, lprev) arrive in LDS in
- *    the same round trip as the block itself; the 16 P tiles (4 a wave,
- *    held in registers until every wave has read lprev) and the 10
- *    lower P P^T tiles are dealt to the 4 waves in turn; P goes through
- *    f.
- *  - Wave 0 then sweeps the columns two at a time: lane r holds row r
- *    of the block (a[c], c <= r; its upper part is never read). At step
- *    j every lane reads the 2 x 2 pivot block [p q; q s] of columns j,
- *    j + 1 from lanes j and j + 1 (cross-lane reads), forms 1 / sqrt(p),
- *    l21 = q / sqrt(p) and 1 / sqrt(s - l21^2), then
+ *    the same round trip as the block itself (all loads before the first
+ *    LDS store: 16.5k -> 6.6k cycles); wave w holds the P tiles of rows
+ *    16 w .. in registers until every wave has read lprev; P goes through
+ *    f; the 10 lower P P^T tiles are dealt to the 4 waves, three chains a
+ *    wave at once (14.6k -> 10k cycles for both products).
+ *  - The block is then factored 16 columns at a time, without LDS round
+ *    trips inside: in wave 0 lane r holds row r of the 16 columns. At
+ *    step j every lane reads the 2 x 2 pivot block [p q; q s] of columns
+ *    j, j + 1 from their lanes (cross-lane reads), forms 1 / sqrt(p), l21 =
+ *    q / sqrt(p) and 1 / sqrt(s - l21^2), then
  *        L[r][j] = a[j] / sqrt(p),
  *        L[r][j + 1] = (a[j + 1] - L[r][j] l21) / sqrt(s - l21^2)
- *    on and below the pivots (0 above); both columns go to LDS (lc)
- *    and each lane applies the rank-2 update
- *        a[c] -= L[r][j] L[c][j] + L[r][j + 1] L[c][j + 1]   (c > j + 1).
- *    The step's dependent chain (cross-lane reads, two roots, one LDS
- *    round trip, the update of the next pivots) thus serves two
- *    columns.
- *  - Wave 1, beside it and a step behind, runs the forward substitution
- *    of L X = I column by column: lane k holds column k of T (the
- *    identity at first),
- *        T[j][k] /= L[j][j],  T[c][k] -= L[c][j] T[j][k]   (c > j),
- *    taking column j from lc once wave 0 has counted it (an LDS counter,
- *    released at the start of wave 0's next step). Each wave holds 64
- *    values a lane, so a step's column reads (16-byte loads, every lane
- *    the same address) are issued together before its updates.
- *  - All threads store the factor from lc in rows; the inverse is stored
- *    from wave 1's registers (lane k: column k, so each store
- *    instruction writes one row of it).
- * Against the earlier form (1024 threads holding the block in LDS, one
- * barrier per two columns): 59.7 -> 41 us a block at n = 1600 with one
- * column a step. */
+ *    and updates its other columns of the 16 with L[c][j], L[c][j + 1]
+ *    read from lane c. The pivots stay in their lanes for one check at the
+ *    end (a branch a step costs 300 cycles). Both columns go to LDS (lc,
+ *    0 above the pivots). What is right of the 16 columns is updated by
+ *    all waves on the matrix instructions.
+ *  - Beside wave 0, 16 rows behind, waves 1 .. 3 run the forward
+ *    substitution of L X = I in f, 16 columns a wave (wave 0 takes the last
+ *    16 after its factor): within 16 rows in registers, below them on the
+ *    matrix instructions.
+ *  - All threads store factor and inverse in rows.
+ * Bound by one wave's dependent chain, about 750 cycles a column pair. A
+ * block at n = 1600: 41 us with a whole-row sweep of the 64 columns (an LDS
+ * round trip and up to 62 updates a lane each step), 22 us so, of 52k
+ * cycles 7k the loads, 10k the look-ahead, 24k the factor, 11k the last rows
+ * of the inverse, the stores and the release. */
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
     chol_diag_kernel(const double *__restrict__ A, double *__restrict__ L,
                       double *__restrict__ Linv, int n, int k, int nb,
@@ -296,8 +302,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
     } u;
     double (*const lc)[GP_NB] = u.lc;
     __shared__ double dinv[GP_NB];
-    __shared__ int prog;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tid = threadIdx.x, lane = tid & 63, kq = lane >> 4, l16 = lane & 15;
+    const int uw = __builtin_amdgcn_readfirstlane(tid >> 6);
     int bad = 0;
 
     if (ready) {
@@ -318,188 +324,224 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
      * With a look-ahead, its operands come in the same round trip: the
      * block row A[k.., k - 64..] (rows past nb zero) into ar and the
      * previous panel's inverse factor into f. */
+    {
+        double v[16], va[16], vl[16];
+
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-        const int e = tid + 256 * i, r = e >> 6, c = e & 63;
-        const long long row = (long long)(k + min(r, nb - 1)) * n;
-        const double v = A[row + k + min(c, nb - 1)];
+        for (int i = 0; i < 16; i++) {
+            const int e = tid + 256 * i, r = e >> 6, c = e & 63;
 
-        if (lprev) {
-            const double va = A[row + k - GP_NB + c], vl = lprev[e];
-
-            u.ar[r][c] = r < nb ? va : 0.0;
-            f[r][c] = vl;
+            v[i] = A[(long long)(k + min(r, nb - 1)) * n + k + min(c, nb - 1)];
         }
-        s[r][c] = r < nb && c <= r ? v : r == c ? 1.0 : 0.0;
+        if (lprev)
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int e = tid + 256 * i, r = e >> 6, c = e & 63;
+
+                va[i] = A[(long long)(k + min(r, nb - 1)) * n + k - GP_NB + c];
+                vl[i] = lprev[e];
+            }
+        __builtin_amdgcn_sched_barrier(0); /* one round trip, not one a row */
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const int e = tid + 256 * i, r = e >> 6, c = e & 63;
+
+            s[r][c] = r < nb && c <= r ? v[i] : r == c ? 1.0 : 0.0;
+        }
+        if (lprev)
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int e = tid + 256 * i, r = e >> 6, c = e & 63;
+
+                u.ar[r][c] = r < nb ? va[i] : 0.0;
+                f[r][c] = vl[i];
+            }
     }
-    if (tid == 0)
-        prog = 0;
     __syncthreads();
     if (lprev) {
-        const int kq = lane >> 4;
-        gp_d4 pacc[4];
+        gp_d4 pacc[4], acc[3];
 
-        /* P tiles (i, (wave + i) % 4) of this wave, from LDS; lprev is
-         * lower triangular, so tile column tc needs k < 16 (tc + 1). */
+        /* P rows 16 wave .., from LDS; lprev is lower triangular, so tile
+         * column tc needs k < 16 (tc + 1). */
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int tc = (wave + i) & 3;
-            const int ri = 16 * i + (lane & 15), ci = 16 * tc + (lane & 15);
-
+        for (int i = 0; i < 4; i++)
             pacc[i] = (gp_d4){0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-            for (int kk = 0; kk < 16; kk++)
-                if (kk < 4 * (tc + 1))
-                    pacc[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-                        u.ar[ri][4 * kk + kq], f[ci][4 * kk + kq], pacc[i], 0, 0, 0);
+        for (int kk = 0; kk < 16; kk++) {
+            const double av = u.ar[16 * uw + l16][4 * kk + kq];
+
+#pragma unroll
+            for (int tc = kk / 4; tc < 4; tc++)
+                pacc[tc] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                    av, f[16 * tc + l16][4 * kk + kq], pacc[tc], 0, 0, 0);
         }
         __syncthreads(); /* every wave is done reading f */
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int tc = (wave + i) & 3;
-
+        for (int tc = 0; tc < 4; tc++)
 #pragma unroll
             for (int v = 0; v < 4; v++)
-                f[16 * i + kq + 4 * v][16 * tc + (lane & 15)] = pacc[i][v];
+                f[16 * uw + kq + 4 * v][16 * tc + l16] = pacc[tc][v];
+        __syncthreads();
+        /* The 10 lower tiles of P P^T, three a wave at once (the last two
+         * waves' third is the last tile again, not stored). */
+        int tr[3], tc[3];
+
+#pragma unroll
+        for (int t = 0; t < 3; t++) {
+            const int w = min(uw + 4 * t, 9);
+
+            tr[t] = w >= 6 ? 3 : w >= 3 ? 2 : w >= 1 ? 1 : 0;
+            tc[t] = w - tr[t] * (tr[t] + 1) / 2;
+            acc[t] = (gp_d4){0.0, 0.0, 0.0, 0.0};
+        }
+#pragma unroll
+        for (int kk = 0; kk < 16; kk++)
+#pragma unroll
+            for (int t = 0; t < 3; t++)
+                acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(f[16 * tr[t] + l16][4 * kk + kq],
+                                                             f[16 * tc[t] + l16][4 * kk + kq],
+                                                             acc[t], 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < 3; t++) {
+            if (uw + 4 * t > 9)
+                continue;
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int r = 16 * tr[t] + kq + 4 * v, c = 16 * tc[t] + l16;
+
+                if (r < nb && c <= r)
+                    s[r][c] -= acc[t][v];
+            }
         }
         __syncthreads();
-        for (int w = wave; w < 10; w += 4) {
-            const int tr2 = w >= 6 ? 3 : w >= 3 ? 2 : w >= 1 ? 1 : 0;
-            const int tc2 = w - tr2 * (tr2 + 1) / 2;
-            const int r2 = 16 * tr2 + (lane & 15), c2 = 16 * tc2 + (lane & 15);
+    }
+    /* The inverse begins as the identity, in f. */
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        const int e = tid + 256 * i;
+
+        f[e >> 6][e & 63] = (e >> 6) == (e & 63) ? 1.0 : 0.0;
+    }
+    __syncthreads();
+    const int nsub = (nb + GP_SB - 1) / GP_SB;
+
+    for (int sp = 0; sp <= nsub; sp++) {
+        if (uw == 0 && sp < nsub) {
+            /* Columns base .. base + 15: lane r holds its row of them.
+             * Pair j, j + 1: the 2 x 2 pivot block [p q; q s] from lanes
+             * base + j and base + j + 1, p's root, then the second pivot s
+             * - l21^2 and its root. Column j + 1 of a lane is its entry
+             * less its column-j value times l21. Columns past nb are
+             * padding (unit pivot, zero elsewhere) and change nothing. */
+            const int base = GP_SB * sp;
+            double a[GP_SB], piv = 1.0, root = 1.0;
+
+#pragma unroll
+            for (int c = 0; c < GP_SB; c++)
+                a[c] = s[lane][base + c];
+#pragma unroll
+            for (int j = 0; j < GP_SB; j += 2) {
+                const int row = lane - base - j; /* rows below the pivot */
+                const double p = readlane_d(a[j], base + j), q = readlane_d(a[j], base + j + 1);
+                const double sq = readlane_d(a[j + 1], base + j + 1);
+                const double rp = rsqrt_nr(p);
+                const double l21 = q * rp;
+                const double s2 = fma(-l21, l21, sq);
+                const double rs = rsqrt_nr(s2);
+                /* The pivots' own lanes hold p and sq: the same products
+                 * give their roots. Lanes above hold what nothing reads. */
+                const double l0 = a[j] * rp;
+                const double l1 = fma(-l0, l21, a[j + 1]) * rs;
+
+                lc[base + j][lane] = row >= 0 ? l0 : 0.0;
+                lc[base + j + 1][lane] = row >= 1 ? l1 : 0.0;
+                piv = row == 0 ? p : row == 1 ? s2 : piv;
+                root = row == 0 ? rp : row == 1 ? rs : root;
+#pragma unroll
+                for (int c = j + 2; c < GP_SB; c++)
+                    a[c] = fma(-l1, readlane_d(l1, base + c),
+                               fma(-l0, readlane_d(l0, base + c), a[c]));
+            }
+            /* Lane base + c has kept pivot c and its reciprocal root. */
+            const bool mine = lane >= base && lane < base + GP_SB;
+            const unsigned long long neg = __ballot(mine && !(piv > 0.0));
+
+            if (mine)
+                dinv[lane] = root;
+            if (bad == 0 && neg)
+                bad = k + __builtin_ctzll(neg) + 1;
+        }
+        else if (sp > 0) {
+            /* Rows base .. base + 15 of the inverse, 16 columns a wave
+             * (wave 0 takes the last ones, when its factor is done): T[j] /=
+             * L[j][j], T[c] -= L[c][j] T[j] within the rows (every lane a
+             * column, four times over), then the rows below on the matrix
+             * instructions. */
+            const int base = GP_SB * (sp - 1), ct = uw ? uw - 1 : 3;
+
+            if (ct < sp) {
+                const int col = GP_SB * ct + l16;
+                double t[GP_SB];
+
+#pragma unroll
+                for (int c = 0; c < GP_SB; c++)
+                    t[c] = f[base + c][col];
+#pragma unroll
+                for (int j = 0; j < GP_SB; j++) {
+                    t[j] *= dinv[base + j];
+#pragma unroll
+                    for (int c = j + 1; c < GP_SB; c++)
+                        t[c] = fma(-lc[base + j][base + c], t[j], t[c]);
+                }
+                if (lane < 16)
+#pragma unroll
+                    for (int c = 0; c < GP_SB; c++)
+                        f[base + c][col] = t[c];
+                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                for (int rt = sp; rt < nsub; rt++) {
+                    gp_d4 acc = {0.0, 0.0, 0.0, 0.0};
+
+#pragma unroll
+                    for (int kk = 0; kk < 4; kk++)
+                        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                            lc[base + 4 * kk + kq][GP_SB * rt + l16], f[base + 4 * kk + kq][col],
+                            acc, 0, 0, 0);
+#pragma unroll
+                    for (int v = 0; v < 4; v++)
+                        f[GP_SB * rt + kq + 4 * v][col] -= acc[v];
+                }
+            }
+        }
+        __syncthreads();
+        if (sp >= nsub - 1)
+            continue;
+        /* The block's rest: lower 16 x 16 tiles, dealt to the waves. */
+        const int left = nsub - 1 - sp;
+
+        for (int w = uw; w < left * (left + 1) / 2; w += 4) {
+            const int tr = w >= 3 ? 2 : w >= 1 ? 1 : 0, tc = w - tr * (tr + 1) / 2;
+            const int r0 = GP_SB * (sp + 1 + tr), c0 = GP_SB * (sp + 1 + tc);
             gp_d4 acc = {0.0, 0.0, 0.0, 0.0};
 
 #pragma unroll
-            for (int kk = 0; kk < 16; kk++)
-                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(f[r2][4 * kk + kq], f[c2][4 * kk + kq],
-                                                          acc, 0, 0, 0);
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int r = 16 * tr2 + kq + 4 * v, c = 16 * tc2 + (lane & 15);
+            for (int kk = 0; kk < 4; kk++) {
+                const double *col = lc[GP_SB * sp + 4 * kk + kq];
 
-                if (r < nb && c <= r)
-                    s[r][c] -= acc[v];
+                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(col[r0 + l16], col[c0 + l16], acc, 0,
+                                                          0, 0);
             }
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                s[r0 + kq + 4 * v][c0 + l16] -= acc[v];
         }
         __syncthreads();
     }
-    if (wave == 0) {
-        /* The factor: lane r holds row r (a[c], c <= r; its upper part
-         * is never read). Column j of L goes to lc[j], the pivot's
-         * reciprocal root to dinv, then the step count to prog. Above
-         * the pivot L[r][j] = 0 is written too, so lc holds the factor
-         * transposed with zeros above its diagonal. */
-        double a[GP_NB];
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        const int e = tid + 256 * i, r = e >> 6, c = e & 63;
 
-#pragma unroll
-        for (int c = 0; c < GP_NB; c++)
-            a[c] = s[lane][c];
-#pragma unroll
-        for (int j = 0; j < GP_NB; j += 2) {
-            if (j >= nb)
-                continue;
-            /* Columns below j and their roots were written a step ago:
-             * counted now, the release's wait for them costs nothing. */
-            if (j > 0 && lane == 0)
-                __hip_atomic_store(&prog, j, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-            /* Pair j, j + 1: the 2 x 2 pivot block [p q; q s] from lanes j
-             * and j + 1, p's root, then the second pivot s - l21^2 and its
-             * root. Column j + 1 of a lane is its entry less its column-j
-             * value times l21, so one LDS round trip and one rank-2 update
-             * serve both columns. When nb is odd the last step's second
-             * column is a padding column (unit pivot, zero elsewhere),
-             * which leaves the real ones unchanged. */
-            const double p = readlane_d(a[j], j), q = readlane_d(a[j], j + 1);
-            const double sq = readlane_d(a[j + 1], j + 1);
-            const double rp = rsqrt_nr(p);
-            const double l21 = q * rp;
-            const double s2 = fma(-l21, l21, sq);
-            const double rs = rsqrt_nr(s2);
-            const double l0 = lane > j ? a[j] * rp : lane == j ? p * rp : 0.0;
-            const double l1 = lane > j + 1   ? fma(-l0, l21, a[j + 1]) * rs
-                              : lane == j + 1 ? s2 * rs
-                                              : 0.0;
-
-            if (lane == 0 && bad == 0) {
-                if (!(p > 0.0))
-                    bad = k + j + 1;
-                else if (!(s2 > 0.0))
-                    bad = k + j + 2;
-            }
-            lc[j][lane] = l0;
-            lc[j + 1][lane] = l1;
-            if (lane == 0) {
-                dinv[j] = rp;
-                dinv[j + 1] = rs;
-            }
-            /* LDS operations of one wave complete in issue order: these
-             * reads see the columns just written. Both columns are read in
-             * full before the updates, so that the loads overlap. */
-            double c0[GP_NB], c1[GP_NB];
-
-#pragma unroll
-            for (int c = j + 2; c < GP_NB; c++) {
-                c0[c] = lc[j][c];
-                c1[c] = lc[j + 1][c];
-            }
-            __builtin_amdgcn_sched_group_barrier(0x100, 64, 0); /* LDS reads first */
-#pragma unroll
-            for (int c = j + 2; c < GP_NB; c++)
-                a[c] = fma(-l1, c1[c], fma(-l0, c0[c], a[c]));
-        }
-        if (lane == 0)
-            __hip_atomic_store(&prog, nb, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-    }
-    else if (wave == 1) {
-        /* The inverse, a step behind, two columns at a time as wave 0
-         * makes them: lane k holds column k of T (the identity at first),
-         *     T[j][k] /= L[j][j],
-         *     T[j + 1][k] = (T[j + 1][k] - L[j + 1][j] T[j][k]) / L[j + 1][j + 1],
-         * then T[c][k] -= L[c][j] T[j][k] + L[c][j + 1] T[j + 1][k] below,
-         * with columns j, j + 1 of L from lc once wave 0 has counted them
-         * (or all nb columns, when j + 1 is a padding column). The wait is
-         * on wave 0 of the same block, which always counts every column;
-         * it is capped all the same. */
-        double t[GP_NB];
-
-#pragma unroll
-        for (int c = 0; c < GP_NB; c++)
-            t[c] = c == lane ? 1.0 : 0.0;
-#pragma unroll
-        for (int j = 0; j < GP_NB; j += 2) {
-            if (j >= nb)
-                continue;
-            const int need = j + 2 < nb ? j + 2 : nb;
-            int it = 0;
-
-            while (__hip_atomic_load(&prog, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) <
-                       need &&
-                   ++it < (1 << 24))
-                __builtin_amdgcn_s_sleep(1);
-            double c0[GP_NB], c1[GP_NB];
-
-#pragma unroll
-            for (int c = j + 1; c < GP_NB; c++)
-                c0[c] = lc[j][c];
-#pragma unroll
-            for (int c = j + 2; c < GP_NB; c++)
-                c1[c] = lc[j + 1][c];
-            __builtin_amdgcn_sched_group_barrier(0x100, 64, 0);
-            const double tj = t[j] * dinv[j];
-            const double tj1 = fma(-c0[j + 1], tj, t[j + 1]) * dinv[j + 1];
-
-            t[j] = tj;
-            t[j + 1] = tj1;
-#pragma unroll
-            for (int c = j + 2; c < GP_NB; c++)
-                t[c] = fma(-c1[c], tj1, fma(-c0[c], tj, t[c]));
-        }
-        /* Lane k writes column k, one row of the inverse per store. */
-        if (lane < nb)
-#pragma unroll
-            for (int m = 0; m < GP_NB; m++)
-                if (m < nb)
-                    Linv[m * GP_NB + lane] = m >= lane ? t[m] : 0.0;
+        if (r < nb && c < nb)
+            Linv[e] = c <= r ? f[r][c] : 0.0;
     }
     __syncthreads();
     if (tid == 0 && bad && *info == 0)
@@ -552,14 +594,6 @@ __global__ void __launch_bounds__(256)
         X[idx] = 0.0;
 }
 
-/* Panel flag: set by one lane after the launches before it on its stream
- * (the panel's trailing update) have finished; device-coherent store. */
-__global__ void __launch_bounds__(64) gp_mark_kernel(int *flag)
-{
-    if (threadIdx.x == 0)
-        __hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 __global__ void __launch_bounds__(256)
     gp_store_kernel(const double *__restrict__ X, long long nf, float *__restrict__ F)
 {
@@ -569,9 +603,8 @@ __global__ void __launch_bounds__(256)
         F[idx] = (float)X[idx];
 }
 
-static dg_args dg(int M, int N, int K, const double *A, long long a_ri, long long a_rk,
-                  const double *B, long long b_rk, long long b_rj, double *C,
-                  long long c_ri, double alpha, int beta, int lower)
+static dg_args dg(int M, int N, int K, const double *A, int a_ri, int a_rk, const double *B,
+                  int b_rk, int b_rj, double *C, int c_ri, double alpha, int beta, int lower)
 {
     dg_args a = {M, N, K, A, a_ri, a_rk, B, b_rk, b_rj, C, c_ri, alpha, beta, lower, 0};
 
@@ -579,9 +612,10 @@ static dg_args dg(int M, int N, int K, const double *A, long long a_ri, long lon
 }
 
 /* One launch for the problems given (those with no output are skipped);
- * wait, spin_max, info as in dg_set. */
+ * wait, spin_max, info, mark as in dg_set. */
 static void dgemm(hipStream_t s, std::initializer_list<const dg_args *> ps,
-                  const int *wait = nullptr, int spin_max = 0, int *info = nullptr)
+                  const int *wait = nullptr, int spin_max = 0, int *info = nullptr,
+                  int *mark = nullptr)
 {
     dg_set pr;
     int np = 0, tx = 0, ty = 0;
@@ -589,6 +623,7 @@ static void dgemm(hipStream_t s, std::initializer_list<const dg_args *> ps,
     pr.wait = wait;
     pr.spin_max = spin_max;
     pr.info = info;
+    pr.mark = mark;
 
     for (const dg_args *a : ps)
         if (a && a->M > 0 && a->N > 0) {
@@ -614,8 +649,8 @@ extern "C" size_t roma_gp_work_bytes(int n, int d)
 }
 
 /* Test hooks (icoreg_gp_test_wait): the in-kernel waits' poll limit and
- * whether the panel flags are set at all (by the second stream's flag
- * kernel and by the diagonal kernels). With the flags never set and a
+ * whether the panel flags are set at all (by the panels' first launches
+ * and by the diagonal kernels). With the flags never set and a
  * short limit, every waiting kernel gives up at once (info = -1) and
  * still exits, so the give-up path and the caller's recovery can be
  * exercised without a stalled stream. */
@@ -637,12 +672,14 @@ static void gp_solve_run(struct ops *o, cl_mem K, int n, float noise, cl_mem F, 
     double *A, *L, *Li, *Z, *Y, *X;
     int *flags;
     const int nblk = (n + GP_NB - 1) / GP_NB;
-    const long long nd = (long long)n * d, w = (long long)d + n;
+    const long long nd = (long long)n * d;
 
     if (n < 1 || d < 1 || n > 46340)
         icoreg_fatal("%s: invalid sizes n=%d d=%d", op, n, d);
     count32((long long)n * n, op);
-    count32((long long)n * w, op);
+    count32((long long)n * ((long long)d + n), op);
+    const int w = d + n;
+
     need_floats(K, 0, (long long)n * n, op, "K");
     need_floats(F, 0, nd, op, "F");
     need_bytes(work, 0, (long long)roma_gp_work_bytes(n, d), op, "work");
@@ -657,7 +694,7 @@ static void gp_solve_run(struct ops *o, cl_mem K, int n, float noise, cl_mem F, 
     flags = (int *)(X + nd);
     {
         prof_scope ps(o->ocl, op);
-        const long long nn = (long long)n * n, nz = n * w;
+        const long long nn = (long long)n * n, nz = (long long)n * w;
         const long long tot = nn > nz ? nn : nz;
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
 
@@ -716,7 +753,8 @@ static void gp_solve_run(struct ops *o, cl_mem K, int n, float noise, cl_mem F, 
             if (capture)
                 dgemm(s2, {&yb, &panel});
             else
-                dgemm(s2, {&yb, &panel}, dflags + b, spin_max, info_p);
+                dgemm(s2, {&yb, &panel}, dflags + b, spin_max, info_p,
+                      b > 0 && g_set_flags ? flags + b - 1 : nullptr);
             /* X[0 : k + nb] += Minv_b^T Y_F,b: this panel's block row of
              * Minv = L^-1 (Y[k.., d..], zero right of its own identity
              * block) is final once Y_b is. */
@@ -735,8 +773,6 @@ static void gp_solve_run(struct ops *o, cl_mem K, int n, float noise, cl_mem F, 
             }
             else
                 dgemm(s2, {&xacc});
-            if (!capture && g_set_flags)
-                hipLaunchKernelGGL(gp_mark_kernel, dim3(1), dim3(64), 0, s2, flags + b);
             if (capture || b == nblk - 1)
                 hip_check(hipEventRecord(aux_event(o->ocl, 2 * b + 1), s2), "hipEventRecord");
         }
