@@ -384,9 +384,12 @@ conv_split_plan conv_split_choose(const conv_args &a, int ks, int st, int nb, in
     }
     /* Below 96 blocks of 64 channels on 256 CUs the smaller blocks of
      * conv_mfma win (128 -> 64 channels at 128 x 128, 64 blocks: 79 us against
-     * 89; 64 -> 128 at 100 x 100, 98: 65 against 51). */
+     * 89; 64 -> 128 at 100 x 100, 98: 65 against 51). With one chunk of
+     * input channels a block is mostly start and end: more than 32 outputs
+     * need 256 (16 -> 64 at 62 x 370, 96: 31.5 us against 37; 16 -> 128 at 128 x
+     * 128, 128: 31 against 41; 16 -> 64 at 256 x 256, 256: 43 -> 39). */
     p.ok = ks == CS_KS && st == 1 && a.C >= 16 && a.K >= 32 &&
-           8 * blocks * (p.bm / 64) >= 3LL * cus;
+           8 * blocks * (p.bm / 64) >= (a.C < 32 && a.K > 32 ? 8LL : 3LL) * cus;
     return p;
 }
 

@@ -921,16 +921,31 @@ static bool gemm_plan(const gemm_args &g, int bmode, int nb, int cus, int &nfull
  * slower: 4.12 -> 4.23 ms a pair in all). */
 #define GEMM_SPLIT_K 512
 
-static bool gemm_split_ok(const gemm_args &g) { return g.K > GEMM_SPLIT_K; }
+/* Where 64 x 64 tiles are few, a block's time is its loads, and splitting
+ * while staging adds to it: without 16-byte loads below 3 / 8 of the CUs
+ * (148 x 685 x 512 10.2 us against 13.7, 24 x 683 x 1024 9.6 against 12.4, 318
+ * x 675 x 535 13.2 against 14.3; 2896 x 2893 x 3175 1089 -> 514), with them below 1024
+ * products and 48 tiles (397 x 872 x 256 9.9 against 10.4; 398 x 868 x 1379
+ * 23.5 -> 19.1). va, vb: 16-byte loads of A and B. */
+static bool gemm_split_ok(const gemm_args &g, int bmode, int nb, bool va, bool vb, int cus)
+{
+    const long long tiles = (long long)nb * ((g.M + 63) / 64) * ((g.N + 63) / 64);
+
+    if (g.K <= GEMM_SPLIT_K)
+        return false;
+    if (bmode == GEMM_B_CONV)
+        return true;
+    return va && vb ? g.K >= 1024 || tiles >= 48 : 8 * tiles >= 3 * cus;
+}
 
 size_t gemm_part_floats(const gemm_args &g, int bmode, int nb, bool va, bool vb, int cus)
 {
     int nfull, split;
 
-    if (gemm_split_ok(g))
-        return gemm_split_floats(g, bmode, nb, cus);
     va = va && g.K % 4 == 0;
     vb = vb && (bmode == GEMM_B_KN ? g.N % 4 == 0 : g.K % 4 == 0);
+    if (gemm_split_ok(g, bmode, nb, va, vb, cus))
+        return gemm_split_floats(g, bmode, nb, cus);
     if (gemm_smallk_ok(g, bmode, nb, va, vb, cus) || gemm_dma_ok(g, bmode, va, vb) ||
         !gemm_plan(g, bmode, nb, cus, nfull, split))
         return 0;
@@ -945,7 +960,7 @@ void gemm_launch(const gemm_args &g, int bmode, int nb, bool va, bool vb,
      * K x N) a multiple of 4. */
     va = va && g.K % 4 == 0;
     vb = vb && (bmode == GEMM_B_KN ? g.N % 4 == 0 : g.K % 4 == 0);
-    if (gemm_split_ok(g)) {
+    if (gemm_split_ok(g, bmode, nb, va, vb, cus)) {
         gemm_split_launch(g, bmode, nb, va, vb, cus, s);
         return;
     }

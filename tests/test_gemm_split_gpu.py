@@ -30,6 +30,9 @@ SHAPES = [
     # Every tile cut over K (few tiles, long K); the last piece shorter.
     (100, 90, 4100, 1, 1, 0, 1, 0),
     (96, 200, 2052, 0, 1, 3, 0, 1),
+    # No 16-byte loads: 99 and 121 tiles of 64 x 64 (fewer run elsewhere).
+    (700, 520, 577, 1, 1, 2, 1, 0),
+    (650, 701, 1023, 0, 1, 0, 0, 1),
     # 288 tiles of 128 x 128: 256 whole, 32 cut.
     (2304, 2000, 1024, 1, 1, 0, 1, 0),
 ]
@@ -73,7 +76,7 @@ def test_edges(shape, dev, ic):
 def test_rows_that_are_not_finite(transb, dev, ic):
     """Infinities, NaN and values that round to bf16 infinity come out as
     float32 products give them, and leave the other rows alone."""
-    M, N, K = 200, 150, 600
+    M, N, K = 200, 152, 1100
     rng = np.random.default_rng(11)
     a = rng.standard_normal((1, M, K)).astype(np.float32)
     b = rng.standard_normal((1, N, K) if transb else (1, K, N)).astype(np.float32)
