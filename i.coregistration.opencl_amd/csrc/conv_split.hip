@@ -75,7 +75,7 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
     for (int c = 0; c < 8; c++)
         v[c] = m < K && c0 + c < C ? w[((long long)m * C + c0 + c) * kk + t] : 0.0f;
-    split8(v, p[0], p[1], p[2]);
+    split8(v, 1.0f, p[0], p[1], p[2]);
 #pragma unroll
     for (int k = 0; k < 3; k++)
         wp[((q * 3 + k) * 2 + i) * 64 + lane] = p[k];
@@ -174,7 +174,7 @@ __global__ void __launch_bounds__(256 * WM, WM)
                 v[c] = poff[q] != CS_OOB && c0 + c < C ? x : 0.0f;
             }
         }
-        split8(v, h, m, l);
+        split8(v, 1.0f, h, m, l);
         if (at[q] >= 0) {
             d[at[q]] = h;
             d[PLANE + at[q]] = m;

@@ -3,14 +3,15 @@
 /* The float32 GEMM of long sums: C = act(alpha A op(B) + bias) + R with every
  * operand value split exactly into three bf16 parts (split.h) and six
  * v_mfma_f32_32x32x16_bf16 products a 32 x 32 x 16 step, accumulated in
- * float32.
+ * float32. The scale that keeps every operand's bits (split.h) is a multiply
+ * a staged value: 159 -> 161 us on the first shape below.
  *
  * What bounds it: the matrix cores and the power they draw. Six bf16
  * products take 192 cycles where eight v_mfma_f32_32x32x2f32 take 512; on
  * random operands the bare instruction stream holds 1.81 PFLOP/s of bf16
  * (the clock falls from 2.4 to about 1.8 GHz), 302 TFLOP/s of float32
  * work, and a large bf16 library product 1.13 PFLOP/s. What the kernel
- * adds to the stream: 5.5 vector instructions a staged value for the split
+ * adds to the stream: 6.5 vector instructions a staged value for the split
  * and the LDS traffic of three parts, both in proportion to the tile's
  * sides, against matrix work in proportion to its area; hence the largest
  * tile that still gives the CUs equal shares.
@@ -31,8 +32,8 @@
  *    come out as float32 products give them.
  *
  * Measured on an MI355X against the kernel on v_mfma_f32_32x32x2f32
- * (gemm.hip): 3202 x 4096 x 1024 with bias and GELU 238.5 -> 160.0 us (113 ->
- * 168 TFLOP/s of float32 work), 3202 x 1024 x 4096 232 -> 174 us, 1140 x
+ * (gemm.hip): 3202 x 4096 x 1024 with bias and GELU 238.5 -> 161.4 us (113 ->
+ * 166 TFLOP/s of float32 work), 3202 x 1024 x 4096 232 -> 174 us, 1140 x
  * 11664 x 1140 (B given K x N) 265 -> 185 us; error against 64-bit sums at K
  * = 1024 6.4e-7 -> 2.1e-7. One block of a CU's two computes while the other
  * stages; 128 x 256 tiles of 4 x 64 x 128 waves ran 146 us on the first shape
@@ -279,7 +280,7 @@ __global__ void __launch_bounds__(T::NT, T::OCC) gemm_split_kernel(const gemm_ar
             const int q = tid + NT * e, row = q / CH;
             const int at = row * CH + ((q % CH) ^ ((row >> SW) & (CH - 1)));
 
-            split8(ra[e], h, m, l);
+            split8(ra[e], SPLIT_UP, h, m, l);
             if (has_a) {
                 as[at] = h;
                 as[PA + at] = m;
@@ -292,7 +293,7 @@ __global__ void __launch_bounds__(T::NT, T::OCC) gemm_split_kernel(const gemm_ar
             const int ch = MODE == GEMM_B_NK ? q % CH : q / BN;
             const int at = row * CH + (ch ^ ((row >> SW) & (CH - 1)));
 
-            split8(rb[e], h, m, l);
+            split8(rb[e], SPLIT_UP, h, m, l);
             if (has_b) {
                 bs[at] = h;
                 bs[PB + at] = m;
@@ -379,7 +380,7 @@ __global__ void __launch_bounds__(T::NT, T::OCC) gemm_split_kernel(const gemm_ar
 
 #pragma unroll
             for (int r = 0; r < 16; r++) {
-                acc[i][j][r] += low[i][j][r];
+                acc[i][j][r] = (acc[i][j][r] + low[i][j][r]) * SPLIT_DOWN;
                 z = fmaf(acc[i][j][r], 0.0f, z);
             }
             if (__any(z != 0.0f))

@@ -477,7 +477,7 @@ __global__ void __launch_bounds__(64 * ATT_NW, ND == 4 ? 1 : 3)
                        ? Q[(long long)qi * a.ldq + dd] * (a.scale * 1.4426950408889634f)
                        : 0.0f;
         }
-        split8(x, q[st][0], q[st][1], q[st][2]);
+        split8(x, 1.0f, q[st][0], q[st][1], q[st][2]);
     }
 #pragma unroll
     for (int t = 0; t < ND; t++)
@@ -539,7 +539,7 @@ __global__ void __launch_bounds__(64 * ATT_NW, ND == 4 ? 1 : 3)
                 const int e = tid + NT * i, key = e / CH;
                 const int at = key * CH + ((e % CH) ^ (key / RW % CH));
 
-                split8(kr[i], x, y, z);
+                split8(kr[i], 1.0f, x, y, z);
                 ks[at] = x;
                 ks[PK + at] = y;
                 ks[2 * PK + at] = z;
@@ -551,7 +551,7 @@ __global__ void __launch_bounds__(64 * ATT_NW, ND == 4 ? 1 : 3)
                 const int e = vt + NT * i, dd = e % DP;
                 const int at = dd * 4 + ((e / DP) ^ (dd >> 2 & 3));
 
-                split8(vr[i], x, y, z);
+                split8(vr[i], 1.0f, x, y, z);
                 vs[at] = x;
                 vs[PK + at] = y;
                 vs[2 * PK + at] = z;
@@ -658,7 +658,7 @@ __global__ void __launch_bounds__(64 * ATT_NW, ND == 4 ? 1 : 3)
 #pragma unroll
             for (int j = 0; j < 8; j++)
                 x[j] = p[8 * u + j];
-            split8(x, pp[0], pp[1], pp[2]);
+            split8(x, 1.0f, pp[0], pp[1], pp[2]);
 #pragma unroll
             for (int tt = 0; tt < ND; tt++) {
                 const int dd = tt * 32 + col;

@@ -115,3 +115,26 @@ def test_sums_of_squares_are_not_biased(dev, ic):
     shift = np.mean(np.diag(g) / want - 1)
     print(f"[gemm split] mean shift {shift:.2e}", flush=True)
     assert abs(shift) <= U / 2
+
+
+@pytest.mark.parametrize("transb", [0, 1])
+@pytest.mark.parametrize("ea,eb", [(-112, 60), (60, -116), (-120, 0), (-126, 120), (120, -145),
+                                   (-20, -100), (38, 38), (60, 60)])
+def test_magnitudes(ea, eb, transb, dev, ic):
+    """Operands of every size, subnormal ones included, keep their 24 bits:
+    of values of about 2^ea and 2^eb the sums' rms error is that of the
+    float32 additions, U of a partial sum (rms at most the sum's) for each of
+    K / 8 + 16, of random sign: U sqrt((K / 8 + 16) / 3). A part lost to
+    bf16's range shows as 2^-22 of the sum or more."""
+    M, N, K = 200, 136, 1100
+    print(f"[gemm split] magnitudes 2^{ea} 2^{eb}", flush=True)
+    rng = np.random.default_rng(K + ea + 7 * eb)
+    a = np.ldexp(rng.standard_normal((1, M, K)), ea).astype(np.float32)
+    b = np.ldexp(rng.standard_normal((1, N, K) if transb else (1, K, N)), eb).astype(np.float32)
+    got = run(dev, ic, a, b, (M, N, K, transb, 1, 0, 0, 0), 1.0, np.zeros(N, np.float32),
+              np.zeros((1, M, N), np.float32))[0]
+    bt = (np.swapaxes(b, 1, 2) if transb else b).astype(np.float64)
+    want = (a.astype(np.float64) @ bt)[0]
+    rms = np.linalg.norm(got - want) / np.linalg.norm(want)
+    print(f"[gemm split] rms error {rms:.2e}", flush=True)
+    assert rms <= U * ((K / 8 + 16) / 3) ** 0.5
