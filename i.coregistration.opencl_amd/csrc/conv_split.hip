@@ -52,7 +52,7 @@ static __device__ __forceinline__ __amdgpu_buffer_rsrc_t cs_rsrc(const float *p,
                                              0x00020000);
 }
 
-/* 16-byte operands of the filters: [64-channel block][16 input channels]
+/* 16-byte operands of the filters, scaled as the input is (split.h): [64-channel block][16 input channels]
  * [tap][part][32-channel half][lane]. Lane l holds output channel l % 32 of
  * the half, input channels 8 (l / 32) .. + 7; zeros past K and C. One
  * thread per (block, slice, tap, half, lane). */
@@ -75,7 +75,7 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
     for (int c = 0; c < 8; c++)
         v[c] = m < K && c0 + c < C ? w[((long long)m * C + c0 + c) * kk + t] : 0.0f;
-    split8(v, 1.0f, p[0], p[1], p[2]);
+    split8(v, SPLIT_UP, p[0], p[1], p[2]);
 #pragma unroll
     for (int k = 0; k < 3; k++)
         wp[((q * 3 + k) * 2 + i) * 64 + lane] = p[k];
@@ -174,7 +174,7 @@ __global__ void __launch_bounds__(256 * WM, WM)
                 v[c] = poff[q] != CS_OOB && c0 + c < C ? x : 0.0f;
             }
         }
-        split8(v, 1.0f, h, m, l);
+        split8(v, SPLIT_UP, h, m, l);
         if (at[q] >= 0) {
             d[at[q]] = h;
             d[PLANE + at[q]] = m;
@@ -288,7 +288,7 @@ __global__ void __launch_bounds__(256 * WM, WM)
 
 #pragma unroll
             for (int r = 0; r < 16; r++) {
-                acc[i][j][r] += low[i][j][r];
+                acc[i][j][r] = (acc[i][j][r] + low[i][j][r]) * SPLIT_DOWN;
                 z = fmaf(acc[i][j][r], 0.0f, z);
             }
             if (__any(z != 0.0f)) {

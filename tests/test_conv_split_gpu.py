@@ -90,3 +90,24 @@ def test_values_that_are_not_finite(dev, ic):
     fine = np.isfinite(ref)
     size = np.maximum(np.abs(ref[fine]), 4)
     assert np.max(np.abs(got[fine] - ref[fine]) / size) <= 1e-5
+
+
+@pytest.mark.parametrize("ex,ew", [(-112, 60), (60, -116), (-120, 0), (-126, 120), (110, -145),
+                                   (38, 38), (60, 60)])
+def test_magnitudes(ex, ew, dev, ic):
+    """Inputs and filters of every size, subnormal ones included, keep their
+    24 bits: the sums' rms error is that of the float32 additions, U of a
+    partial sum (rms at most the sum's) for each of n / 8 + 16, of random
+    sign: U sqrt((n / 8 + 16) / 3). A part lost to bf16's range shows as 2^-22
+    of the sum or more."""
+    c = (1, 32, 40, 128, 200, 2, 0, 0)
+    print(f"[conv split] magnitudes 2^{ex} 2^{ew}", flush=True)
+    x, w, b, _ = tensors(c, 3)
+    x = np.ldexp(x.astype(np.float64), ex).astype(np.float32)
+    w = np.ldexp(w.astype(np.float64), ew).astype(np.float32)
+    b[:] = 0
+    got = run(dev, ic, c, x, w, b, None)
+    ref, _ = want(c, x, w, b, None)
+    rms = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    print(f"[conv split] rms error {rms:.2e}", flush=True)
+    assert rms <= U * ((25 * c[1] / 8 + 16) / 3) ** 0.5
