@@ -50,6 +50,7 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 #define ATT_KT 32 /* keys per tile */
 #define ATT_NW 4  /* waves per block, 32 queries each */
 #define ATT_TAU 8.0f /* lazy rescaling threshold, base-2 units */
+#define ATT_QUP 0x1p32f /* scale of the queries split into bf16 parts */
 #define ATT_PF 2     /* LDS operand reads ahead of their MFMA */
 
 /* Registers <- the key tile from key k0 (zeros past Nk and d), 16-byte
@@ -427,6 +428,12 @@ __global__ void __launch_bounds__(64 * ATT_NW) attention_kernel(const att_args a
  * 65 .. 96 channels stay on the fp32 block: rows of 12 chunks would not
  * spread over the banks this way.
  *
+ * Values and probabilities are scaled as split.h says. Queries are scaled by
+ * ATT_QUP and keys not: scores need absolute precision, and a query of 2^95
+ * and above (after the softmax scale) is no longer finite, so what keys under
+ * 2^-110 lose, at most 2^-134 each, moves a score by at most d 2^-38. The
+ * scale leaves the scores in the exponential's multiply-add.
+ *
  * If a sum is not finite (an infinity or NaN among the operands has no
  * split), the block runs again on the fp32 instructions. */
 template <int ND, bool VEC, bool MASK>
@@ -464,6 +471,7 @@ __global__ void __launch_bounds__(64 * ATT_NW, ND == 4 ? 1 : 3)
     split_u4 q[2 * ND][3];
     floatx16 o[ND];
     float m = -INFINITY, l = 0.0f;
+    bool kept = !MASK && t0 < t1;
 
 #pragma unroll
     for (int st = 0; st < 2 * ND; st++) {
@@ -474,7 +482,8 @@ __global__ void __launch_bounds__(64 * ATT_NW, ND == 4 ? 1 : 3)
             const int dd = st * 16 + half * 8 + j;
 
             x[j] = qi < a.Nq && dd < d
-                       ? Q[(long long)qi * a.ldq + dd] * (a.scale * 1.4426950408889634f)
+                       ? Q[(long long)qi * a.ldq + dd] *
+                             (a.scale * 1.4426950408889634f * ATT_QUP)
                        : 0.0f;
         }
         split8(x, 1.0f, q[st][0], q[st][1], q[st][2]);
@@ -551,7 +560,7 @@ __global__ void __launch_bounds__(64 * ATT_NW, ND == 4 ? 1 : 3)
                 const int e = vt + NT * i, dd = e % DP;
                 const int at = dd * 4 + ((e / DP) ^ (dd >> 2 & 3));
 
-                split8(vr[i], 1.0f, x, y, z);
+                split8(vr[i], SPLIT_UP, x, y, z);
                 vs[at] = x;
                 vs[PK + at] = y;
                 vs[2 * PK + at] = z;
@@ -604,6 +613,7 @@ __global__ void __launch_bounds__(64 * ATT_NW, ND == 4 ? 1 : 3)
 
                 if (MASK)
                     keep = keep && a.kmask[min(kk, Nk - 1)] != 0;
+                kept = kept || keep;
                 p[r] = keep ? s[r] : -INFINITY;
                 mx = fmaxf(mx, p[r]);
             }
@@ -615,7 +625,7 @@ __global__ void __launch_bounds__(64 * ATT_NW, ND == 4 ? 1 : 3)
                 mx = fmaxf(mx, p[r]);
             }
         }
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64)) * (1.0f / ATT_QUP);
         const bool need = mx > m + ATT_TAU;
 
         if (__any(need)) {
@@ -637,7 +647,7 @@ __global__ void __launch_bounds__(64 * ATT_NW, ND == 4 ? 1 : 3)
 
 #pragma unroll
             for (int r = 0; r < 16; r++) {
-                p[r] = __builtin_amdgcn_exp2f(p[r] - ref);
+                p[r] = __builtin_amdgcn_exp2f(fmaf(p[r], 1.0f / ATT_QUP, -ref));
                 sum += p[r];
             }
         }
@@ -658,7 +668,7 @@ __global__ void __launch_bounds__(64 * ATT_NW, ND == 4 ? 1 : 3)
 #pragma unroll
             for (int j = 0; j < 8; j++)
                 x[j] = p[8 * u + j];
-            split8(x, 1.0f, pp[0], pp[1], pp[2]);
+            split8(x, SPLIT_UP, pp[0], pp[1], pp[2]);
 #pragma unroll
             for (int tt = 0; tt < ND; tt++) {
                 const int dd = tt * 32 + col;
@@ -685,7 +695,9 @@ __global__ void __launch_bounds__(64 * ATT_NW, ND == 4 ? 1 : 3)
 #pragma unroll
             for (int r = 0; r < 16; r++)
                 z = fmaf(o[tt][r], 0.0f, z);
-        if (__syncthreads_or(z != 0.0f)) {
+        /* No probability at all for keys that were kept: their scores lie
+         * below the range. */
+        if (__syncthreads_or(z != 0.0f || (l == 0.0f && __any(kept)))) {
             att_block_f32<ND, false, MASK>(a, (float *)lds, bx, by, bz, ny);
             return;
         }
@@ -693,7 +705,7 @@ __global__ void __launch_bounds__(64 * ATT_NW, ND == 4 ? 1 : 3)
     if (qi >= a.Nq)
         return;
     if (!a.part_o) {
-        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+        const float inv = l > 0.0f ? 1.0f / l * SPLIT_DOWN : 0.0f;
         float *out = a.O + bi * a.bo + (long long)qi * a.ldo + (long long)h * d;
 
 #pragma unroll
@@ -715,8 +727,8 @@ __global__ void __launch_bounds__(64 * ATT_NW, ND == 4 ? 1 : 3)
 #pragma unroll
             for (int g = 0; g < 4; g++)
                 *(float4 *)(out + tt * 32 + g * 8 + half * 4) =
-                    make_float4(o[tt][4 * g], o[tt][4 * g + 1], o[tt][4 * g + 2],
-                                o[tt][4 * g + 3]);
+                    make_float4(o[tt][4 * g] * SPLIT_DOWN, o[tt][4 * g + 1] * SPLIT_DOWN,
+                                o[tt][4 * g + 2] * SPLIT_DOWN, o[tt][4 * g + 3] * SPLIT_DOWN);
         if (half == 0)
             a.part_ml[row] = make_float2(m, l);
     }

@@ -113,3 +113,41 @@ def test_values_that_are_not_finite(d, dev, ic):
     rows = np.delete(np.arange(Nq), 9)
     assert np.allclose(got[rows, 2], clean[0, rows, 2], rtol=0, atol=1e-4)
     assert np.array_equal(got[:, 3], clean[0, :, 3])
+
+
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("eq,ek,ev", [(-116, 116, 0), (90, -90, 0), (0, 0, -116), (0, 0, 60),
+                                      (-110, 110, -120)])
+def test_powers_of_two(eq, ek, ev, d, dev, ic):
+    """Scaling queries against keys, or values, by powers of two changes no
+    bit but the exponents (no value or result here is subnormal)."""
+    print(f"[attention split] 2^{eq} 2^{ek} 2^{ev} d={d}", flush=True)
+    rng = np.random.default_rng(d)
+    # Magnitudes in [1, 8), values positive: the scaled operands and the
+    # results are normal numbers.
+    q, k, v = ((rng.uniform(1, 8, (1, n, 2, d)) * rng.choice([-1, 1], (1, n, 2, d))).astype(np.float32)
+               for n in (70, 300, 300))
+    v = np.abs(v)
+    scale = float(np.float32(0.1 / np.sqrt(d)))
+    base = run(dev, ic, q, k, v, scale)
+    got = run(dev, ic, np.ldexp(q, eq), np.ldexp(k, ek), np.ldexp(v, ev), scale)
+    assert np.array_equal(got, np.ldexp(base, ev))
+
+
+@pytest.mark.parametrize("masked", [0, 1])
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_scores_far_below_zero(d, masked, dev, ic):
+    """Every score near -2^120: each query takes its best key's values."""
+    print(f"[attention split] far below zero d={d} masked={masked}", flush=True)
+    rng = np.random.default_rng(d)
+    q, k, v = (rng.uniform(0.5, 2, (1, n, 2, d)).astype(np.float32) for n in (70, 300, 300))
+    mask = (rng.random(300) < 0.5).astype(np.uint8) if masked else None
+    if masked:
+        mask[:64] = 0
+    got = run(dev, ic, np.ldexp(q, 60), np.ldexp(-k, 60), v, 0.125, 0, mask)
+    s = -np.einsum("qhd,khd->hqk", q[0].astype(np.float64), k[0].astype(np.float64))
+    if masked:
+        s[:, :, mask == 0] = -np.inf
+    best = s.argmax(-1)
+    for h in range(2):
+        assert np.allclose(got[0, :, h], v[0, best[h], h], rtol=4 * U, atol=0)
