@@ -38,12 +38,12 @@ bool conv_direct_supported(int kh, int kw, int sy, int sx, int dy, int dx,
 bool conv_direct_fits(long long in_floats, long long w_floats);
 
 /* Bytes of work memory conv_direct_launch needs for a (filters in operand
- * order and partial sums; 0: none); the caller passes that much as a.part,
- * or NULL for the kernels that need none. */
-size_t conv_direct_part_bytes(const conv_args &a, int ks, int stride, int nb, int cus);
+ * order and partial sums; 0: none); the caller passes that much as a.part.
+ * bf16: 5 x 5 layers may run on the bf16 instructions (conv_split.hip). */
+size_t conv_direct_part_bytes(const conv_args &a, int ks, int stride, int nb, int cus, bool bf16);
 
 void conv_direct_launch(const conv_args &a, int ks, int stride, int nb,
-                        int cus, hipStream_t s);
+                        int cus, hipStream_t s, bool bf16);
 
 /* The direct 5 x 5 convolution, stride 1, on the bf16 matrix instructions
  * (conv_split.hip): channels a block, tile width, pieces over the input

@@ -678,7 +678,7 @@ static size_t split_filter_bytes(const conv_args &m)
     return (conv_split_weight_bytes(m.K, m.C) + 255) & ~(size_t)255;
 }
 
-size_t conv_direct_part_bytes(const conv_args &a, int ks, int stride, int nb, int cus)
+size_t conv_direct_part_bytes(const conv_args &a, int ks, int stride, int nb, int cus, bool bf16)
 {
     if (a.C == 1 && !a.mean && a.K <= C1_MAXK && a.K * ks * ks <= C1_MAXW)
         return 0;
@@ -687,7 +687,7 @@ size_t conv_direct_part_bytes(const conv_args &a, int ks, int stride, int nb, in
     direct_plan p = plan_direct(a, ks, nb, cus);
     size_t fewk = 0, filters = 0;
 
-    if (sp.ok) {
+    if (bf16 && sp.ok) {
         p.kmain = m.K;
         p.split = sp.split;
         filters = split_filter_bytes(m);
@@ -729,14 +729,14 @@ static void launch_cfg(const conv_args &a, const direct_plan &p, int nb, int cus
 }
 
 template <int KS, int ST>
-static void launch_ks(const conv_args &a, int nb, int cus, hipStream_t s)
+static void launch_ks(const conv_args &a, int nb, int cus, hipStream_t s, bool bf16)
 {
     constexpr int NJ = KS == 3 ? 1 : 2;
     const conv_args m = split_main(a, KS);
     const conv_split_plan sp = conv_split_choose(m, KS, ST, nb, cus);
-    direct_plan p = plan_direct(a, KS, nb, cus);
+    const direct_plan p = plan_direct(a, KS, nb, cus);
 
-    if (sp.ok && a.part) {
+    if (bf16 && sp.ok) {
         /* Filters, then the partial sums. */
         conv_args b = a, c = m;
 
@@ -751,9 +751,6 @@ static void launch_ks(const conv_args &a, int nb, int cus, hipStream_t s)
             launch_fewk<KS, ST>(b, m.K, a.K - m.K, nb, cus, s);
         return;
     }
-    if (!a.part)
-        p.split = 1;
-
     if (p.bm == 128) {
         if (p.tw == 16)
             launch_cfg<KS, ST, 128, 16, NJ>(a, p, nb, cus, s);
@@ -768,7 +765,7 @@ static void launch_ks(const conv_args &a, int nb, int cus, hipStream_t s)
 }
 
 void conv_direct_launch(const conv_args &a, int ks, int stride, int nb,
-                        int cus, hipStream_t s)
+                        int cus, hipStream_t s, bool bf16)
 {
     if (a.C == 1 && !a.mean && a.K <= C1_MAXK && a.K * ks * ks <= C1_MAXW) {
         const dim3 grid((unsigned)(((long long)a.Ho * a.Wo + 255) / 256), 1, nb);
@@ -784,11 +781,11 @@ void conv_direct_launch(const conv_args &a, int ks, int stride, int nb,
         return;
     }
     if (ks == 3 && stride == 1)
-        launch_ks<3, 1>(a, nb, cus, s);
+        launch_ks<3, 1>(a, nb, cus, s, bf16);
     else if (ks == 3)
-        launch_ks<3, 2>(a, nb, cus, s);
+        launch_ks<3, 2>(a, nb, cus, s, bf16);
     else if (stride == 1)
-        launch_ks<5, 1>(a, nb, cus, s);
+        launch_ks<5, 1>(a, nb, cus, s, bf16);
     else
-        launch_ks<5, 2>(a, nb, cus, s);
+        launch_ks<5, 2>(a, nb, cus, s, bf16);
 }

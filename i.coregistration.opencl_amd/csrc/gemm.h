@@ -59,13 +59,16 @@ struct gemm_args {
 bool gemm_shape_ok(const gemm_args &g, int bmode);
 
 /* Launch on stream s over nb batches on a device of cus CUs. va/vb:
- * 16-byte vector loads allowed for A / B (every row start aligned). */
+ * 16-byte vector loads allowed for A / B (every row start aligned). bf16:
+ * long sums may run on the bf16 instructions (gemm_split.hip), if they need
+ * no part or have it. */
 void gemm_launch(const gemm_args &g, int bmode, int nb, bool va, bool vb,
-                 int cus, hipStream_t s);
+                 int cus, hipStream_t s, bool bf16 = true);
 
 /* Floats of part that gemm_launch's kernel for g needs (0: it runs without
  * pieces). */
-size_t gemm_part_floats(const gemm_args &g, int bmode, int nb, bool va, bool vb, int cus);
+size_t gemm_part_floats(const gemm_args &g, int bmode, int nb, bool va, bool vb, int cus,
+                        bool bf16 = true);
 
 /* gemm_launch and gemm_part_floats for the products of the bf16
  * instructions (gemm_split.hip). */

@@ -938,13 +938,14 @@ static bool gemm_split_ok(const gemm_args &g, int bmode, int nb, bool va, bool v
     return va && vb ? g.K >= 1024 || tiles >= 48 : 8 * tiles >= 3 * cus;
 }
 
-size_t gemm_part_floats(const gemm_args &g, int bmode, int nb, bool va, bool vb, int cus)
+size_t gemm_part_floats(const gemm_args &g, int bmode, int nb, bool va, bool vb, int cus,
+                        bool bf16)
 {
     int nfull, split;
 
     va = va && g.K % 4 == 0;
     vb = vb && (bmode == GEMM_B_KN ? g.N % 4 == 0 : g.K % 4 == 0);
-    if (gemm_split_ok(g, bmode, nb, va, vb, cus))
+    if (bf16 && gemm_split_ok(g, bmode, nb, va, vb, cus))
         return gemm_split_floats(g, bmode, nb, cus);
     if (gemm_smallk_ok(g, bmode, nb, va, vb, cus) || gemm_dma_ok(g, bmode, va, vb) ||
         !gemm_plan(g, bmode, nb, cus, nfull, split))
@@ -953,14 +954,14 @@ size_t gemm_part_floats(const gemm_args &g, int bmode, int nb, bool va, bool vb,
 }
 
 void gemm_launch(const gemm_args &g, int bmode, int nb, bool va, bool vb,
-                 int cus, hipStream_t s)
+                 int cus, hipStream_t s, bool bf16)
 {
     /* 16-byte loads need every four-float group wholly inside or wholly
      * past the matrix edge: K (A, and B given N x K) or N (B given
      * K x N) a multiple of 4. */
     va = va && g.K % 4 == 0;
     vb = vb && (bmode == GEMM_B_KN ? g.N % 4 == 0 : g.K % 4 == 0);
-    if (gemm_split_ok(g, bmode, nb, va, vb, cus)) {
+    if (bf16 && gemm_split_ok(g, bmode, nb, va, vb, cus)) {
         gemm_split_launch(g, bmode, nb, va, vb, cus, s);
         return;
     }

@@ -29,10 +29,22 @@ extern "C" void ops_init(struct ops *o, struct ocl_backend *ocl)
 
 namespace icoreg {
 
+/* True while the library's stream is recorded into a graph. */
+static bool recording(struct ops *o)
+{
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+
+    hip_check(hipStreamIsCapturing(stream_of(o->ocl), &st), "hipStreamIsCapturing");
+    return st != hipStreamCaptureStatusNone;
+}
+
 cl_mem scratch_get(struct ops *o, size_t bytes)
 {
     if (bytes <= o->scratch_bytes && o->scratch)
         return o->scratch;
+    if (recording(o))
+        icoreg_fatal("the ops work buffer cannot grow to %zu bytes while a graph is being recorded",
+                     bytes);
     hip_check(hipStreamSynchronize(stream_of(o->ocl)), "hipStreamSynchronize");
     ocl_release(&o->scratch);
     bytes = (bytes + 0xfffff) & ~(size_t)0xfffff;
@@ -41,16 +53,13 @@ cl_mem scratch_get(struct ops *o, size_t bytes)
     return o->scratch;
 }
 
-/* scratch_get, or NULL where it would have to grow while the stream is
- * recorded into a graph (nothing can be allocated then). */
-static cl_mem scratch_or_null(struct ops *o, size_t bytes)
+/* True if scratch_get can give bytes: not where the buffer would have to
+ * grow while the stream is recorded into a graph. The kernels on the bf16
+ * instructions take more work memory than the fp32 ones, which a recording
+ * then takes in their place (and whose own need it refuses if short). */
+static bool scratch_fits(struct ops *o, size_t bytes)
 {
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-
-    if (bytes <= o->scratch_bytes && o->scratch)
-        return o->scratch;
-    hip_check(hipStreamIsCapturing(stream_of(o->ocl), &st), "hipStreamIsCapturing");
-    return st == hipStreamCaptureStatusNone ? scratch_get(o, bytes) : NULL;
+    return bytes <= o->scratch_bytes || !recording(o);
 }
 
 } // namespace icoreg
@@ -200,12 +209,17 @@ extern "C" void ops_gemm(struct ops *o, int M, int N, int K, struct opnd A,
         gemm_args g = gemm_make(op, M, N, K, A, B, transb, C, nb, nb1, bias, biasrow, R, roff,
                                 alpha, act, slope);
         /* Partial sums of cut tiles, when the grid leaves CUs uneven. */
-        const size_t pf = gemm_part_floats(g, bmode, nb, vec_ok(A), vec_ok(B), o->ocl->cu_count);
+        const bool va = vec_ok(A), vb = vec_ok(B);
+        const int cus = o->ocl->cu_count;
+        size_t pf = gemm_part_floats(g, bmode, nb, va, vb, cus);
+        const bool bf16 = scratch_fits(o, pf * sizeof(float));
 
+        if (!bf16)
+            pf = gemm_part_floats(g, bmode, nb, va, vb, cus, false);
         if (pf)
-            g.part = fptr(scratch_or_null(o, pf * sizeof(float)));
+            g.part = fptr(scratch_get(o, pf * sizeof(float)));
         prof_scope ps(o->ocl, "gemm");
-        gemm_launch(g, bmode, nb, vec_ok(A), vec_ok(B), o->ocl->cu_count, stream_of(o->ocl));
+        gemm_launch(g, bmode, nb, va, vb, cus, stream_of(o->ocl), bf16);
         launch_check("gemm");
     }
     ICOREG_API_END
@@ -598,15 +612,15 @@ static void conv_impl(struct ops *o, int nb, cl_mem in, long long in_stride,
         a.slope = slope;
         a.split = 1;
         a.part = nullptr;
-        {
-            const size_t pb = conv_direct_part_bytes(a, g->kh, g->sy, nb, o->ocl->cu_count);
+        size_t pb = conv_direct_part_bytes(a, g->kh, g->sy, nb, o->ocl->cu_count, true);
+        const bool bf16 = scratch_fits(o, pb);
 
-            if (pb)
-                a.part = fptr(scratch_or_null(o, pb));
-        }
+        if (!bf16)
+            pb = conv_direct_part_bytes(a, g->kh, g->sy, nb, o->ocl->cu_count, false);
+        if (pb)
+            a.part = fptr(scratch_get(o, pb));
         prof_scope ps(o->ocl, "conv_direct");
-        conv_direct_launch(a, g->kh, g->sy, nb, o->ocl->cu_count,
-                           stream_of(o->ocl));
+        conv_direct_launch(a, g->kh, g->sy, nb, o->ocl->cu_count, stream_of(o->ocl), bf16);
         launch_check("conv_direct");
         return;
     }

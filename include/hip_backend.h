@@ -84,8 +84,11 @@ void ocl_init(struct ocl_backend *ocl, const char *device_opt,
  * ocl_graph_begin and ocl_graph_end are recorded, not run, into a HIP
  * graph that ocl_graph_launch replays on the stream. Calls that allocate,
  * read, write or synchronise are errors while recording (run the work
- * once before recording, so that the ops work buffer has its size). The
- * graph holds the buffer addresses of the recording. */
+ * once before recording, so that the ops work buffer has its size: an
+ * operation whose kernels all need more is an error, and a matrix product or
+ * 5 x 5 convolution that has a kernel for which the buffer suffices is
+ * recorded with that one, whose sums may round differently from those of an
+ * eager call). The graph holds the buffer addresses of the recording. */
 void ocl_graph_begin(struct ocl_backend *ocl);
 void *ocl_graph_end(struct ocl_backend *ocl);
 void ocl_graph_launch(struct ocl_backend *ocl, void *graph);
