@@ -16,9 +16,10 @@
  * sides, against matrix work in proportion to its area; hence the largest
  * tile that still gives the CUs equal shares.
  *
- *  - A block stages BK = 16 or 32 k of both operands: buffer loads through
- *    windows over the tile's rows (past the edge they read 0) into
- *    registers a slice ahead, split there, three [row][k] planes in LDS.
+ *  - A block stages 32 k of both operands: buffer loads through windows
+ *    over the tile's rows (past the edge they read 0) into registers a
+ *    slice ahead, split there, three [row][k] planes in LDS (one buffer and
+ *    two barriers a slice: the CU's other blocks fill the gap).
  *    A lane's MFMA operand is eight consecutive k: one ds_read_b128.
  *  - The 16-byte chunks of a row are stored XORed with bits of the row so
  *    that the 16 rows a quarter of a read touches lie in 64 different
@@ -48,17 +49,16 @@
 /* Most pieces a tile is cut into over K. */
 #define SPLIT_MAX 8
 
-/* Tile shape: BM x BN outputs, BK of K a slice, WM x WN waves, NBUF LDS
- * buffers (1: two barriers a slice, other blocks of the CU fill the gap;
- * 2: one barrier, the next slice is split beside the products). */
-template <int BM_, int BN_, int BK_, int WM_, int WN_, int NBUF_, int OCC_> struct split_tile {
-    static constexpr int BM = BM_, BN = BN_, BK = BK_, WM = WM_, WN = WN_, NBUF = NBUF_;
-    static constexpr int OCC = OCC_; /* waves a SIMD at least */
+#define SPLIT_BK 32 /* k of a slice */
+
+/* Tile shape: BM x BN outputs, WM x WN waves, at least OCC of them a SIMD. */
+template <int BM_, int BN_, int WM_, int WN_, int OCC_> struct split_tile {
+    static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, OCC = OCC_;
     static constexpr int NT = 64 * WM * WN, TM = BM / WM / 32, TN = BN / WN / 32;
 };
-typedef split_tile<128, 128, 32, 2, 4, 1, 4> split_m;
-typedef split_tile<64, 128, 32, 2, 2, 1, 3> split_s;
-typedef split_tile<64, 64, 32, 2, 2, 1, 4> split_xs;
+typedef split_tile<128, 128, 2, 4, 4> split_m;
+typedef split_tile<64, 128, 2, 2, 3> split_s;
+typedef split_tile<64, 64, 2, 2, 4> split_xs;
 
 /* Row and column tile of tile number t: down the columns where there are
  * fewer rows of tiles, so that the tiles an XCD's L2 serves together share
@@ -141,15 +141,13 @@ __device__ __forceinline__ floatx16 split_tile_f32(const gemm_args &g, const flo
 template <class T, int MODE, bool VEC>
 __global__ void __launch_bounds__(T::NT, T::OCC) gemm_split_kernel(const gemm_args g)
 {
-    constexpr int BM = T::BM, BN = T::BN, BK = T::BK, WN = T::WN, NT = T::NT;
+    constexpr int BM = T::BM, BN = T::BN, BK = SPLIT_BK, WN = T::WN, NT = T::NT;
     constexpr int TM = T::TM, TN = T::TN, WR = BM / T::WM, WC = BN / WN;
-    constexpr int CH = BK / 8;       /* 16-byte chunks of a row and plane */
-    constexpr int SW = CH == 4 ? 2 : 3; /* row bits that order the chunks */
+    constexpr int CH = BK / 8;                /* 16-byte chunks of a row and plane */
     constexpr int PA = BM * CH, PB = BN * CH; /* chunks a plane */
-    constexpr int AC = (PA + NT - 1) / NT, BC = (PB + NT - 1) / NT;
-    static_assert((PA % NT == 0 || PA < NT) && (PB % NT == 0 || PB < NT) && BN % 64 == 0,
-                  "tile shape");
-    __shared__ split_u4 lds[T::NBUF][3 * (PA + PB)];
+    constexpr int AC = PA / NT, BC = PB / NT; /* chunks a thread */
+    static_assert(PA % NT == 0 && PB % NT == 0 && BN % 64 == 0, "tile shape");
+    __shared__ split_u4 lds[3 * (PA + PB)];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -177,7 +175,6 @@ __global__ void __launch_bounds__(T::NT, T::OCC) gemm_split_kernel(const gemm_ar
     static_assert(NT % BN == 0, "a thread keeps its column of B");
     /* Chunk q of a plane: row q / CH, chunk q % CH; B given K x N: column
      * q % BN, chunk q / BN (the same for a whole wave). */
-    const bool has_a = PA >= NT || tid < PA, has_b = PB >= NT || tid < PB;
     unsigned aoff[AC], boff[BC];
     float ra[AC][8], rb[BC][8];
     floatx16 acc[TM][TN], low[TM][TN];
@@ -207,15 +204,12 @@ __global__ void __launch_bounds__(T::NT, T::OCC) gemm_split_kernel(const gemm_ar
      * window's end and read 0; k past K read the next row of all but the
      * last one and are set to 0. */
     auto fetch = [&](int k0) {
-        if (has_a) {
-            const __amdgpu_buffer_rsrc_t wa =
-                gemm_rsrc(Ab + k0, ((rows_a - 1) * lda + K - k0) * 4);
+        const __amdgpu_buffer_rsrc_t wa = gemm_rsrc(Ab + k0, ((rows_a - 1) * lda + K - k0) * 4);
 
 #pragma unroll
-            for (int e = 0; e < AC; e++)
-                split_load8<VEC>(wa, aoff[e], ra[e]);
-        }
-        if (MODE == GEMM_B_NK && has_b) {
+        for (int e = 0; e < AC; e++)
+            split_load8<VEC>(wa, aoff[e], ra[e]);
+        if (MODE == GEMM_B_NK) {
             const __amdgpu_buffer_rsrc_t wb =
                 gemm_rsrc(Bb + k0, ((cols_b - 1) * ldb + K - k0) * 4);
 
@@ -223,7 +217,7 @@ __global__ void __launch_bounds__(T::NT, T::OCC) gemm_split_kernel(const gemm_ar
             for (int e = 0; e < BC; e++)
                 split_load8<VEC>(wb, boff[e], rb[e]);
         }
-        else if (MODE == GEMM_B_CONV && has_b) {
+        else if (MODE == GEMM_B_CONV) {
             /* A thread's column is the same in all its chunks (BN divides
              * the block's threads). */
             const int p = n0 + tid % BN;
@@ -239,7 +233,7 @@ __global__ void __launch_bounds__(T::NT, T::OCC) gemm_split_kernel(const gemm_ar
                                             p < N && kr + i < K);
             }
         }
-        else if (has_b) {
+        else {
             /* A window a row of B: the base and its size are scalars. */
 #pragma unroll
             for (int e = 0; e < BC; e++) {
@@ -272,37 +266,33 @@ __global__ void __launch_bounds__(T::NT, T::OCC) gemm_split_kernel(const gemm_ar
             }
         }
     };
-    auto stash = [&](split_u4 *as) {
-        split_u4 *bs = as + 3 * PA, h, m, l;
+    auto stash = [&]() {
+        split_u4 *const as = lds, *const bs = as + 3 * PA, h, m, l;
 
 #pragma unroll
         for (int e = 0; e < AC; e++) {
             const int q = tid + NT * e, row = q / CH;
-            const int at = row * CH + ((q % CH) ^ ((row >> SW) & (CH - 1)));
+            const int at = row * CH + ((q % CH) ^ ((row >> 2) & (CH - 1)));
 
             split8(ra[e], SPLIT_UP, h, m, l);
-            if (has_a) {
-                as[at] = h;
-                as[PA + at] = m;
-                as[2 * PA + at] = l;
-            }
+            as[at] = h;
+            as[PA + at] = m;
+            as[2 * PA + at] = l;
         }
 #pragma unroll
         for (int e = 0; e < BC; e++) {
             const int q = tid + NT * e, row = MODE == GEMM_B_NK ? q / CH : q % BN;
             const int ch = MODE == GEMM_B_NK ? q % CH : q / BN;
-            const int at = row * CH + (ch ^ ((row >> SW) & (CH - 1)));
+            const int at = row * CH + (ch ^ ((row >> 2) & (CH - 1)));
 
             split8(rb[e], SPLIT_UP, h, m, l);
-            if (has_b) {
-                bs[at] = h;
-                bs[PB + at] = m;
-                bs[2 * PB + at] = l;
-            }
+            bs[at] = h;
+            bs[PB + at] = m;
+            bs[2 * PB + at] = l;
         }
     };
-    auto compute = [&](const split_u4 *as) {
-        const split_u4 *bs = as + 3 * PA;
+    auto compute = [&]() {
+        const split_u4 *const as = lds, *const bs = as + 3 * PA;
 
 #pragma unroll
         for (int ks = 0; ks < BK / 16; ks++) {
@@ -316,7 +306,7 @@ __global__ void __launch_bounds__(T::NT, T::OCC) gemm_split_kernel(const gemm_ar
 
                     a[p][i] = __builtin_bit_cast(
                         split_b8,
-                        as[p * PA + row * CH + ((2 * ks + kh) ^ ((row >> SW) & (CH - 1)))]);
+                        as[p * PA + row * CH + ((2 * ks + kh) ^ ((row >> 2) & (CH - 1)))]);
                 }
 #pragma unroll
                 for (int j = 0; j < TN; j++) {
@@ -324,7 +314,7 @@ __global__ void __launch_bounds__(T::NT, T::OCC) gemm_split_kernel(const gemm_ar
 
                     b[p][j] = __builtin_bit_cast(
                         split_b8,
-                        bs[p * PB + row * CH + ((2 * ks + kh) ^ ((row >> SW) & (CH - 1)))]);
+                        bs[p * PB + row * CH + ((2 * ks + kh) ^ ((row >> 2) & (CH - 1)))]);
                 }
             }
             /* Parts (h, m, l) = (0, 1, 2); hh into acc, the other five
@@ -346,30 +336,13 @@ __global__ void __launch_bounds__(T::NT, T::OCC) gemm_split_kernel(const gemm_ar
 
     if (kt0 < kt1) {
         fetch(kt0 * BK);
-        if (T::NBUF == 1) {
-            for (int kt = kt0; kt < kt1; kt++) {
-                __syncthreads();
-                stash(lds[0]);
-                __syncthreads();
-                if (kt + 1 < kt1)
-                    fetch((kt + 1) * BK);
-                compute(lds[0]);
-            }
-        }
-        else {
-            stash(lds[0]);
-            if (kt0 + 1 < kt1)
-                fetch((kt0 + 1) * BK);
-            for (int kt = kt0; kt < kt1; kt++) {
-                const int cur = (kt - kt0) & 1;
-
-                __syncthreads();
-                if (kt + 1 < kt1)
-                    stash(lds[(cur ^ 1) % T::NBUF]);
-                if (kt + 2 < kt1)
-                    fetch((kt + 2) * BK);
-                compute(lds[cur % T::NBUF]);
-            }
+        for (int kt = kt0; kt < kt1; kt++) {
+            __syncthreads();
+            stash();
+            __syncthreads();
+            if (kt + 1 < kt1)
+                fetch((kt + 1) * BK);
+            compute();
         }
     }
 #pragma unroll
