@@ -28,9 +28,10 @@
  *    hh's at the end: added to the large sums one by one they round away
  *    (mm of a sum of squares did, which moved such sums by -1.3e-7 of their
  *    value), and hh's sums take a sixth of the roundings.
- *  - Tiles whose sums are not all finite are formed again from the float32
- *    operands on v_mfma_f32_32x32x2f32, so infinities, NaN and overflow
- *    come out as float32 products give them.
+ *  - 32 x 32 tiles whose sums are not all finite are formed again on
+ *    v_mfma_f32_32x32x2f32 by a second pass of the block over its unsplit
+ *    slices, so infinities, NaN and overflow come out as float32 products
+ *    give them, at about the time of the fp32 kernel on top.
  *
  * Measured on an MI355X against the kernel on v_mfma_f32_32x32x2f32
  * (gemm.hip): 3202 x 4096 x 1024 with bias and GELU 238.5 -> 161.4 us (113 ->
@@ -109,33 +110,6 @@ __device__ __forceinline__ float split_gather(const gemm_args &g, const float *B
             v = v >= 0.0f ? v : g.gate[c] * v;
     }
     return in ? v : 0.0f;
-}
-
-/* One 32 x 32 tile over k in [k0, k1) from the float32 operands. */
-template <int MODE>
-__device__ __forceinline__ floatx16 split_tile_f32(const gemm_args &g, const float *A,
-                                                   const float *B, int row, int col, int k0,
-                                                   int k1, int kh)
-{
-    floatx16 acc;
-
-    for (int r = 0; r < 16; r++)
-        acc[r] = 0.0f;
-#pragma unroll 1
-    for (int k = k0 + kh; k < k1 + kh; k += 2) {
-        const bool in = k < k1;
-        const float a = in && row < g.M ? A[(long long)row * g.lda + k] : 0.0f;
-        float b = 0.0f;
-
-        if (MODE == GEMM_B_CONV)
-            b = split_gather(g, B, in ? k : 0, col / g.wo * g.sy - g.py,
-                             col % g.wo * g.sx - g.px, in && col < g.N);
-        else if (in && col < g.N)
-            b = MODE == GEMM_B_NK ? B[(long long)col * g.ldb + k] : B[(long long)k * g.ldb + col];
-
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc, 0, 0, 0);
-    }
-    return acc;
 }
 
 template <class T, int MODE, bool VEC>
@@ -345,6 +319,8 @@ __global__ void __launch_bounds__(T::NT, T::OCC) gemm_split_kernel(const gemm_ar
             compute();
         }
     }
+    unsigned redo = 0; /* bit i TN + j: a sum of the tile is not finite */
+
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
@@ -356,11 +332,64 @@ __global__ void __launch_bounds__(T::NT, T::OCC) gemm_split_kernel(const gemm_ar
                 acc[i][j][r] = (acc[i][j][r] + low[i][j][r]) * SPLIT_DOWN;
                 z = fmaf(acc[i][j][r], 0.0f, z);
             }
-            if (__any(z != 0.0f))
-                acc[i][j] = split_tile_f32<MODE>(g, A, B, m0 + wm * WR + i * 32 + r32,
-                                                 n0 + wn * WC + j * 32 + r32, kt0 * BK,
-                                                 min(kt1 * BK, K), kh);
+            redo |= __any(z != 0.0f) ? 1u << (i * TN + j) : 0u;
         }
+    if (__syncthreads_or((int)redo)) {
+        /* Those tiles again, on the float32 instructions: the block stages
+         * its slices unsplit, [row][k], rows one float apart in the banks. */
+        constexpr int P = BK + 1;
+        static_assert((BM + BN) * P <= 4 * 3 * (PA + PB), "the slices fit");
+        float *const as = (float *)lds, *const bs = as + BM * P;
+
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+#pragma unroll
+                for (int r = 0; r < 16; r++)
+                    low[i][j][r] = 0.0f;
+        for (int kt = kt0; kt < kt1; kt++) {
+            fetch(kt * BK);
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < AC; e++) {
+                const int q = tid + NT * e;
+
+#pragma unroll
+                for (int x = 0; x < 8; x++)
+                    as[q / CH * P + q % CH * 8 + x] = ra[e][x];
+            }
+#pragma unroll
+            for (int e = 0; e < BC; e++) {
+                const int q = tid + NT * e, row = MODE == GEMM_B_NK ? q / CH : q % BN;
+                const int ch = MODE == GEMM_B_NK ? q % CH : q / BN;
+
+#pragma unroll
+                for (int x = 0; x < 8; x++)
+                    bs[row * P + ch * 8 + x] = rb[e][x];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++)
+                    if (redo >> (i * TN + j) & 1u) {
+                        const float *a = as + (wm * WR + i * 32 + r32) * P + kh;
+                        const float *b = bs + (wn * WC + j * 32 + r32) * P + kh;
+
+#pragma unroll
+                        for (int k = 0; k < BK; k += 2)
+                            low[i][j] =
+                                __builtin_amdgcn_mfma_f32_32x32x2f32(a[k], b[k], low[i][j], 0, 0, 0);
+                    }
+        }
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+                if (redo >> (i * TN + j) & 1u)
+                    acc[i][j] = low[i][j];
+    }
     if (piece >= 0) {
         /* The piece's sums: float4 e = 4 (i TN + j) + r / 4 of every
          * thread of the block, threads together. */
