@@ -24,8 +24,8 @@
  *    G taps at a time, a group ahead, through registers (by LDS DMA the
  *    compiler puts a full wait before the next LDS read: 728 us for DISK's
  *    last layer; read by every wave straight into its operands: 807 us).
- * Tiles whose sums are not all finite are formed again from the float32
- * values (v_mfma_f32_32x32x2f32).
+ * Tiles whose sums are not all finite are formed again by a second pass of
+ * the block over the unsplit values (v_mfma_f32_32x32x2f32).
  *
  * Measured on an MI355X against conv_mfma (conv.hip): 80 -> 129 channels at
  * 512 x 512 with normalisation (its 129th channel on conv_fewk_kernel both
@@ -184,6 +184,12 @@ __global__ void __launch_bounds__(256 * WM, WM)
     /* Group g of slice s: chunk tid + NT q of it into fr[q]. */
     constexpr int FL = (G * FT * 64 + NT - 1) / NT;
     split_u4 fr[FL];
+    /* All threads have a chunk q of n. Blocks of 64 channels then go without
+     * a branch, between which a load may wait for the one before it (DISK's
+     * 64-channel layers at 256 x 256 134 - 157 us with them); blocks of 128
+     * keep it, their schedule is better with it (80 -> 129 channels at 512 x
+     * 512 692 us against 723). */
+    auto all = [](int q, int n) { return WM == 1 && NT * (q + 1) <= n; };
     auto filters = [&](int s, int g) {
         const int n = min(G, KK - g * G) * FT * 64;
 
@@ -192,7 +198,7 @@ __global__ void __launch_bounds__(256 * WM, WM)
             const int c = tid + NT * q, t = c / (FT * 64), r = c % (FT * 64);
             const int mb = r / 384;
 
-            if (c < n)
+            if (all(q, n) || c < n)
                 fr[q] = wp[((((long long)blockIdx.y * WM + mb) * nc + s) * KK + g * G + t) * 384 +
                            r % 384];
         }
@@ -202,7 +208,7 @@ __global__ void __launch_bounds__(256 * WM, WM)
 
 #pragma unroll
         for (int q = 0; q < FL; q++)
-            if (tid + NT * q < n)
+            if (all(q, n) || tid + NT * q < n)
                 d[tid + NT * q] = fr[q];
     };
 
@@ -272,6 +278,96 @@ __global__ void __launch_bounds__(256 * WM, WM)
         }
     }
 
+    unsigned redo = 0; /* bit 2 i + j: a sum of the tile is not finite */
+
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            float z = 0.0f;
+
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                acc[i][j][r] = (acc[i][j][r] + low[i][j][r]) * SPLIT_DOWN;
+                z = fmaf(acc[i][j][r], 0.0f, z);
+            }
+            redo |= __any(z != 0.0f) ? 1u << (2 * i + j) : 0u;
+        }
+    if (__syncthreads_or((int)redo)) {
+        /* Those tiles again, on the float32 instructions: the 16 channels of
+         * a slice unsplit, planes half the banks apart, and a row of taps'
+         * filters at a time, [tap][output][16 channels and one]. */
+        constexpr int PP = (PH * PW + 31) / 64 * 64 + 32, FR = 64 * WM, FP = 17;
+        static_assert(PP >= PH * PW && 16 * PP * 4 <= (int)sizeof(lds) &&
+                          KS * FR * FP * 4 <= (int)sizeof(fil),
+                      "slice and filters fit");
+        float *const ps = (float *)lds, *const fs = (float *)fil;
+
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int r = 0; r < 16; r++)
+                    low[i][j][r] = 0.0f;
+        for (int s = s0; s < s1; s++) {
+            __syncthreads();
+#pragma unroll 2
+            for (int e = tid; e < 16 * PH * PW; e += NT) {
+                const int c = e / (PH * PW), p = e % (PH * PW), k = min(s * 16 + c, C - 1);
+                const int y = iy0 + p / PW, x = ix0 + p % PW;
+                const bool in_ = s * 16 + c < C && (unsigned)y < (unsigned)H &&
+                                 (unsigned)x < (unsigned)W;
+                float v = in[k * HW + (in_ ? (long long)y * W + x : 0)];
+
+                if (a.mean) {
+                    v = (v - a.mean[k]) * a.rstd[k];
+                    if (a.gate)
+                        v = v >= 0.0f ? v : a.gate[k] * v;
+                }
+                ps[c * PP + p] = in_ ? v : 0.0f;
+            }
+#pragma unroll 1
+            for (int ky = 0; ky < KS; ky++) {
+                if (ky > 0)
+                    __syncthreads();
+#pragma unroll 4
+                for (int e = tid; e < FR * 16 * KS; e += NT) {
+                    const int m = e / (16 * KS), c = e % (16 * KS) / KS, x = e % KS;
+                    const int k = blockIdx.y * FR + m;
+
+                    fs[(x * FR + m) * FP + c] =
+                        k < a.K && s * 16 + c < C
+                            ? a.w[((long long)k * C + s * 16 + c) * KK + ky * KS + x]
+                            : 0.0f;
+                }
+                __syncthreads();
+#pragma unroll 1
+                for (int x = 0; x < KS; x++) {
+                    const float *f = fs + (x * FR + wm * 64 + r32) * FP + kh;
+                    const float *b = ps + kh * PP + (pr + ky) * PW + pc + x;
+
+#pragma unroll
+                    for (int c = 0; c < 16; c += 2)
+#pragma unroll
+                        for (int i = 0; i < 2; i++)
+#pragma unroll
+                            for (int j = 0; j < 2; j++)
+                                if (redo >> (2 * i + j) & 1u)
+                                    low[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                                        f[i * 32 * FP + c], b[c * PP + j * RJ * PW], low[i][j], 0,
+                                        0, 0);
+                }
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+                if (redo >> (2 * i + j) & 1u)
+                    acc[i][j] = low[i][j];
+    }
+
     const bool whole = a.split == 1;
     float *out = whole ? a.out + (long long)img * a.out_stride
                        : a.part + ((long long)piece * (gridDim.z / a.split) + img) * a.K * a.Ho *
@@ -284,40 +380,7 @@ __global__ void __launch_bounds__(256 * WM, WM)
 
 #pragma unroll
         for (int i = 0; i < 2; i++) {
-            float z = 0.0f, bias[16];
-
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                acc[i][j][r] = (acc[i][j][r] + low[i][j][r]) * SPLIT_DOWN;
-                z = fmaf(acc[i][j][r], 0.0f, z);
-            }
-            if (__any(z != 0.0f)) {
-                /* k = channel * taps + tap, from the float32 values. */
-                const int m = m0 + i * 32 + r32, k1 = min(s1 * 16, C) * KK;
-                split_f16x d;
-
-#pragma unroll
-                for (int r = 0; r < 16; r++)
-                    d[r] = 0.0f;
-#pragma unroll 1
-                for (int k = s0 * 16 * KK + kh; k < k1 + kh; k += 2) {
-                    const int kc = min(k, k1 - 1), c = kc / KK, t = kc - c * KK;
-                    const int y = oy - a.pad + t / KS, x = ox - a.pad + t % KS;
-                    const bool ok = k < k1 && inside && (unsigned)y < (unsigned)H &&
-                                    (unsigned)x < (unsigned)W;
-                    float b = in[c * HW + (ok ? (long long)y * W + x : 0)];
-
-                    if (a.mean) {
-                        b = (b - a.mean[c]) * a.rstd[c];
-                        if (a.gate)
-                            b = b >= 0.0f ? b : a.gate[c] * b;
-                    }
-                    d = __builtin_amdgcn_mfma_f32_32x32x2f32(
-                        k < k1 && m < a.K ? a.w[(long long)m * C * KK + kc] : 0.0f,
-                        ok ? b : 0.0f, d, 0, 0, 0);
-                }
-                acc[i][j] = d;
-            }
+            float bias[16];
             const int mr = m0 + i * 32 + kh * 4;
 
 #pragma unroll

@@ -7,6 +7,8 @@ Bound: as for the products of tests/test_gemm_split_gpu.py, 2^-24 (n / 8 +
 16) sum |w x| over the n = 25 C terms, plus the input normalisation's
 rounding (three float32 steps a value, 3 * 2^-24 |w x|)."""
 
+import time
+
 import numpy as np
 import pytest
 import torch
@@ -111,3 +113,63 @@ def test_magnitudes(ex, ew, dev, ic):
     rms = np.linalg.norm(got - ref) / np.linalg.norm(ref)
     print(f"[conv split] rms error {rms:.2e}", flush=True)
     assert rms <= U * ((25 * c[1] / 8 + 16) / 3) ** 0.5
+
+
+# Pieces over three slices of channels; normalised, 128 outputs a block, 16
+# and 32 pixels wide tiles.
+@pytest.mark.parametrize("c", [(1, 36, 40, 160, 165, 2, 0, 0), (1, 33, 128, 200, 330, 2, 1, 0),
+                               (1, 34, 200, 120, 384, 1, 1, 0)], ids=str)
+def test_values_that_are_not_finite_again(c, dev, ic):
+    """Infinities, NaN and values without a split among the inputs and the
+    filters, in the first and the last channels and at corners, come out as
+    float32 products give them; outputs they do not reach are unmoved."""
+    print(f"[conv split] not finite {c}", flush=True)
+    x, w, b, v = tensors(c, 11)
+    n, C, K, H, W, pad, norm, act = c
+    x[0, 3, 0, 0] = np.inf
+    x[0, C - 1, H // 2, 70] = np.nan
+    x[0, 16, H - 1, W - 1] = 2e38  # above 2^104
+    x[0, 5, 30, 100] = -np.inf
+    w[7, 3, 2, 2] = 0              # inf * 0
+    w[K - 1, 2, 1, 4] = np.inf     # one output channel
+    w[:, 16] *= 0.25               # no output overflows
+    got = run(dev, ic, c, x, w, b, v)
+    with np.errstate(over="ignore", invalid="ignore"):
+        ref, size = want(c, x, w, b, v)
+        ref = ref.astype(np.float32)
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)])
+    fine = np.isfinite(ref)
+    assert fine[0, :K - 1].mean() > 0.9
+    # The fp32 instructions round each of the n terms.
+    assert np.max(np.abs(got[fine] - ref[fine]) / (U * (25 * C + 19) * size[fine])) <= 1
+
+
+def test_cost_of_values_that_are_not_finite(dev, ic):
+    """A second pass on the fp32 instructions, whose kernel takes about twice
+    the bf16 one's time: an image of nothing but NaN costs at most five times
+    (a pass that gathers each value took 11)."""
+    C, K, H, W = 64, 128, 256, 256
+    w = np.ones((K, C, 5, 5), np.float32)
+    Wt, B, out = dev.upload(w), dev.zeros(K), dev.zeros(K * H * W)
+    g = ic.geom(5, 5, 1, 1, 2, 2, 1, 1, 1)
+
+    def best(value):
+        X = dev.upload(np.full((C, H, W), value, np.float32))
+        times = []
+        for _ in range(6):
+            dev.finish()
+            t = time.perf_counter()
+            for _ in range(5):
+                dev.api.ops_conv2d_batch(dev.po, 1, X.mem, C * H * W, C, H, W, Wt.mem, B.mem, K,
+                                         ic.C.byref(g), None, None, None, 0, 0.0, out.mem,
+                                         K * H * W)
+            dev.finish()
+            times.append(time.perf_counter() - t)
+        return min(times)
+
+    print("[conv split] cost", flush=True)
+    clean, nan = best(1.0), best(np.nan)
+    print(f"[conv split] {nan / clean:.2f} times", flush=True)
+    assert np.isnan(dev.read(out)).all()
+    assert nan <= 5 * clean
