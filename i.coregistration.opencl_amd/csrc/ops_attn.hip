@@ -409,13 +409,15 @@ __global__ void __launch_bounds__(64 * ATT_NW) attention_kernel(const att_args a
  * is key 16 u + 8 (j / 4) + 4 h + j % 4, so the split probabilities are the
  * second product's operands as they stand. 16-byte chunks are stored XORed
  * with row bits, 16 rows to 64 banks. A score's 5 small products per 16
- * channels are summed before the large ones. The output's small products of
- * 16 keys are summed apart and added once: one by one onto a sum over all
- * keys they round away, all one way where the values have one sign (mean
- * shift at 4000 keys -1.1e-8, so 2e-9; rms error at 128 keys, 32 channels
- * 1.46e-7 against the fp32 block's 1.05e-7, so 0.95e-7; 2 x 16 heads of 64,
- * 1601 tokens 152 -> 155 us; summed apart over a whole tile the
- * probabilities' parts need registers that spill: 157).
+ * channels are summed before the large ones. The output's small products
+ * have accumulators of their own: one by one onto a sum over all keys they
+ * round away, all one way where the values have one sign (mean shift at 4000
+ * keys -1.1e-8, so 3e-9; rms error at 128 keys, 32 channels 1.46e-7 against
+ * the fp32 block's 1.05e-7, so 0.9e-7). With 64 channels these accumulators
+ * would spill (160 us on the first shape below); there the small products of
+ * 16 keys are summed apart and added once (155 us; of 32 keys 157). With 128,
+ * adding so took 124 us for 8 heads, 1600 tokens, accumulators 110 (101 with
+ * no sums apart).
  *
  * Per 32 keys, 32 queries and 64 channels 48 products (1536 cycles) run
  * beside 16 exponentials and 32 splits a lane (about 1200 cycles of vector
@@ -475,7 +477,10 @@ __global__ void __launch_bounds__(64 * ATT_NW, ND == 4 ? 1 : 3)
     const int vt = APART ? tid - PK : tid;
     float kr[NL][8], vr[NL][8];
     split_u4 q[2 * ND][3];
-    floatx16 o[ND];
+    /* The output's small products: of all keys (LOW), or of 16 at a time
+     * where 16 registers a 32 channels more would spill. */
+    constexpr bool LOW = ND != 2;
+    floatx16 o[ND], low[LOW ? ND : 1];
     float m = -INFINITY, l = 0.0f;
     bool kept = !MASK && t0 < t1;
 
@@ -498,7 +503,7 @@ __global__ void __launch_bounds__(64 * ATT_NW, ND == 4 ? 1 : 3)
     for (int t = 0; t < ND; t++)
 #pragma unroll
         for (int r = 0; r < 16; r++)
-            o[t][r] = 0.0f;
+            o[t][r] = low[LOW ? t : 0][r] = 0.0f;
 
     /* Tile k0 into registers: K chunk e is key e / CH, channels 8 (e % CH)
      * ..; V chunk e channel e % DP, slots 8 (e / DP) .. + 7 (keys that a
@@ -644,8 +649,11 @@ __global__ void __launch_bounds__(64 * ATT_NW, ND == 4 ? 1 : 3)
 #pragma unroll
             for (int tt = 0; tt < ND; tt++)
 #pragma unroll
-                for (int r = 0; r < 16; r++)
+                for (int r = 0; r < 16; r++) {
                     o[tt][r] *= corr;
+                    if (LOW)
+                        low[LOW ? tt : 0][r] *= corr;
+                }
         }
         {
             /* No key kept yet: every score is -infinity, 2^-infinity = 0. */
@@ -679,25 +687,27 @@ __global__ void __launch_bounds__(64 * ATT_NW, ND == 4 ? 1 : 3)
             for (int tt = 0; tt < ND; tt++) {
                 const int dd = tt * 32 + col;
                 split_b8 vf[3];
-                floatx16 low;
+                floatx16 &part = low[LOW ? tt : 0];
 
+                if (!LOW)
 #pragma unroll
-                for (int r = 0; r < 16; r++)
-                    low[r] = 0.0f;
+                    for (int r = 0; r < 16; r++)
+                        part[r] = 0.0f;
 #pragma unroll
                 for (int k = 0; k < 3; k++)
                     vf[k] = __builtin_bit_cast(
                         split_b8, vs[k * PK + dd * 4 + ((2 * u + half) ^ (dd >> 2 & 3))]);
 #pragma unroll
                 for (int w = 0; w < 6; w++) {
-                    floatx16 &c = w == 5 ? o[tt] : low;
+                    floatx16 &c = w == 5 ? o[tt] : part;
 
                     c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
                         vf[pa[w]], __builtin_bit_cast(split_b8, pp[pb[w]]), c, 0, 0, 0);
                 }
+                if (!LOW)
 #pragma unroll
-                for (int r = 0; r < 16; r++)
-                    o[tt][r] += low[r];
+                    for (int r = 0; r < 16; r++)
+                        o[tt][r] += part[r];
             }
         }
         __syncthreads();
@@ -709,8 +719,11 @@ __global__ void __launch_bounds__(64 * ATT_NW, ND == 4 ? 1 : 3)
 #pragma unroll
         for (int tt = 0; tt < ND; tt++)
 #pragma unroll
-            for (int r = 0; r < 16; r++)
+            for (int r = 0; r < 16; r++) {
+                if (LOW)
+                    o[tt][r] += low[LOW ? tt : 0][r];
                 z = fmaf(o[tt][r], 0.0f, z);
+            }
         /* No probability at all for keys that were kept: their scores lie
          * below the range. */
         if (__syncthreads_or(z != 0.0f || (l == 0.0f && __any(kept)))) {
