@@ -727,7 +727,7 @@ __global__ void __launch_bounds__(64 * ATT_NW, ND == 4 ? 1 : 3)
         /* No probability at all for keys that were kept: their scores lie
          * below the range. */
         if (__syncthreads_or(z != 0.0f || (l == 0.0f && __any(kept)))) {
-            att_block_f32<ND, false, MASK>(a, (float *)lds, bx, by, bz, ny);
+            att_block_f32<ND, VEC, MASK>(a, (float *)lds, bx, by, bz, ny);
             return;
         }
     }

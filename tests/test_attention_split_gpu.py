@@ -9,6 +9,8 @@ by that much relatively, and by 4 U for its exponential; the numerator and
 the denominator both carry it. The sum over the keys adds U (Nk / 8 + 16),
 the merge of key ranges and the division 32 U at most, of sum p |v|."""
 
+import time
+
 import numpy as np
 import pytest
 
@@ -174,3 +176,63 @@ def test_positive_values_are_not_biased(d, Nk, dev, ic):
         shift += np.mean(got[:, h] / want - 1) / nh
     print(f"[attention split] mean shift {shift:.2e}", flush=True)
     assert abs(shift) <= U / 16
+
+
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_values_that_are_not_finite_masked(d, dev, ic):
+    """With a key mask: infinities and NaN in keys that are left out change
+    nothing but their block's instructions, except a value's, which meets a
+    probability of zero (0 * NaN) as in fp32; in keys that are kept they come
+    out as without a mask. A key range that is left out whole stays empty."""
+    print(f"[attention split] masked not finite d={d}", flush=True)
+    rng = np.random.default_rng(d + 1)
+    nh, Nq, Nk = 4, 150, 200
+    q, k, v = (rng.standard_normal((1, n, nh, d)).astype(np.float32) for n in (Nq, Nk, Nk))
+    mask = (rng.random(Nk) < 0.6).astype(np.uint8)
+    mask[:64] = 0
+    mask[[150, 160]] = 0, 1
+    scale = float(1.0 / np.sqrt(d))
+    clean = run(dev, ic, q, k, v, scale, 0, mask)[0]
+    k[0, 150, 0, 1] = np.nan   # left out
+    k[0, 10, 0, 2] = np.inf    # left out
+    v[0, 160, 1, 3] = np.inf   # kept
+    v[0, 160, 2, 4] = 1e36     # kept, above 2^104
+    got = run(dev, ic, q, k, v, scale, 0, mask)[0]
+    assert np.allclose(got[:, 0], clean[:, 0], rtol=0, atol=1e-5)
+    assert np.all(got[:, 1, 3] == np.inf)
+    assert np.allclose(np.delete(got[:, 1], 3, 1), np.delete(clean[:, 1], 3, 1), rtol=0, atol=1e-5)
+    s = scale * q[0, :, 2].astype(np.float64) @ k[0, :, 2].astype(np.float64).T
+    s[:, mask == 0] = -np.inf
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    assert np.allclose(got[:, 2, 4], p[:, 160] * 1e36, rtol=1e-4)
+    assert np.array_equal(got[:, 3], clean[:, 3])
+
+
+def test_cost_of_values_that_are_not_finite(dev, ic):
+    """The fp32 block runs after the bf16 one and takes about 1.7 times as
+    long: queries of nothing but NaN cost at most 3.3 times (4 without 16-byte
+    loads)."""
+    nb, n, nh, d = 2, 1601, 8, 128
+    ld = nh * d
+    K, V = (dev.upload(np.ones((nb, n, ld), np.float32)) for _ in range(2))
+    O = dev.zeros(nb * n * ld)
+
+    def best(value):
+        Q = dev.upload(np.full((nb, n, ld), value, np.float32))
+        times = []
+        for _ in range(6):
+            dev.finish()
+            t = time.perf_counter()
+            for _ in range(10):
+                dev.api.ops_attention_batch(dev.po, nb, ic.mat(Q, 0, ld), n * ld, ic.mat(K, 0, ld),
+                                            n * ld, ic.mat(V, 0, ld), n * ld, ic.mat(O, 0, ld),
+                                            n * ld, n, n, nh, d, 0.1, None)
+            dev.finish()
+            times.append(time.perf_counter() - t)
+        return min(times)
+
+    print("[attention split] cost", flush=True)
+    clean, nan = best(1.0), best(np.nan)
+    print(f"[attention split] {nan / clean:.2f} times", flush=True)
+    assert nan <= 3.3 * clean
