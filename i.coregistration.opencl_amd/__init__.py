@@ -241,6 +241,8 @@ SIGNATURES = {
     "icoreg_gp_test_wait": (None, [_I, _I]),
     "icoreg_conv_wino_form": (None, [_I]),
     "icoreg_conv_wino_choice": (_I, [_P, _I, _I, _I, _I, _I]),
+    "icoreg_gemm_choice": (_I, [_O, _I, _I, _I, _I, _I, _I]),
+    "icoreg_conv5_choice": (_I, [_O, _I, _I, _I, _I, _I, _I]),
     "icoreg_roma_gp_retries": (_I, [_P]),
 }
 
@@ -257,7 +259,7 @@ _NO_CHECK = {"ocl_graph_free", "icoreg_set_fatal_mode", "icoreg_last_error", "ic
              "icoreg_roma_set_imagenet", "icoreg_disk_new", "icoreg_disk_buffer",
              "icoreg_roma_last", "disk_topn_work_bytes", "adalam_nearest_work_bytes",
              "icoreg_gp_test_wait", "icoreg_roma_gp_retries", "icoreg_conv_wino_form",
-             "icoreg_conv_wino_choice"}
+             "icoreg_conv_wino_choice", "icoreg_gemm_choice", "icoreg_conv5_choice"}
 
 _lib = None
 

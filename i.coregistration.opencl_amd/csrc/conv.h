@@ -42,6 +42,10 @@ bool conv_direct_fits(long long in_floats, long long w_floats);
  * bf16: 5 x 5 layers may run on the bf16 instructions (conv_split.hip). */
 size_t conv_direct_part_bytes(const conv_args &a, int ks, int stride, int nb, int cus, bool bf16);
 
+/* Pieces over the input channels that conv_direct_launch cuts a 5 x 5, stride
+ * 1 layer of a's sizes into on the bf16 instructions; 0: it runs on others. */
+int conv_direct_choice(const conv_args &a, int nb, int cus);
+
 void conv_direct_launch(const conv_args &a, int ks, int stride, int nb,
                         int cus, hipStream_t s, bool bf16);
 

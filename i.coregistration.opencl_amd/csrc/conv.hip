@@ -678,6 +678,13 @@ static size_t split_filter_bytes(const conv_args &m)
     return (conv_split_weight_bytes(m.K, m.C) + 255) & ~(size_t)255;
 }
 
+int conv_direct_choice(const conv_args &a, int nb, int cus)
+{
+    const conv_split_plan p = conv_split_choose(split_main(a, 5), 5, 1, nb, cus);
+
+    return p.ok ? p.split : 0;
+}
+
 size_t conv_direct_part_bytes(const conv_args &a, int ks, int stride, int nb, int cus, bool bf16)
 {
     if (a.C == 1 && !a.mean && a.K <= C1_MAXK && a.K * ks * ks <= C1_MAXW)

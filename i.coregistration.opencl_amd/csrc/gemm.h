@@ -76,6 +76,10 @@ void gemm_split_launch(const gemm_args &g, int bmode, int nb, bool va, bool vb, 
                        hipStream_t s);
 size_t gemm_split_floats(const gemm_args &g, int bmode, int nb, int cus);
 
+/* What gemm_launch runs a product of g's M, N, K on: 0 the fp32
+ * instructions, 1 the bf16 ones, 2 the bf16 ones with tiles cut over K. */
+int gemm_choice(const gemm_args &g, int bmode, int nb, bool va, bool vb, int cus);
+
 /* True if gemm_launch would run g on the small-product kernel. */
 bool gemm_smallk_ok(const gemm_args &g, int bmode, int nb, bool va, bool vb, int cus);
 

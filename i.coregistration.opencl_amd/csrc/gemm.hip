@@ -938,6 +938,15 @@ static bool gemm_split_ok(const gemm_args &g, int bmode, int nb, bool va, bool v
     return va && vb ? g.K >= 1024 || tiles >= 48 : 8 * tiles >= 3 * cus;
 }
 
+int gemm_choice(const gemm_args &g, int bmode, int nb, bool va, bool vb, int cus)
+{
+    va = va && g.K % 4 == 0;
+    vb = vb && (bmode == GEMM_B_KN ? g.N % 4 == 0 : g.K % 4 == 0);
+    return !gemm_split_ok(g, bmode, nb, va, vb, cus)     ? 0
+           : gemm_split_floats(g, bmode, nb, cus) == 0 ? 1
+                                                         : 2;
+}
+
 size_t gemm_part_floats(const gemm_args &g, int bmode, int nb, bool va, bool vb, int cus,
                         bool bf16)
 {

@@ -460,6 +460,32 @@ extern "C" int icoreg_conv_wino_choice(struct ops *o, int nb, int C, int H, int 
     return wino4_chosen(a, nb, o->ocl->cu_count) ? 4 : 2;
 }
 
+extern "C" int icoreg_gemm_choice(struct ops *o, int M, int N, int K, int b, int nb, int aligned)
+{
+    gemm_args g = {};
+
+    g.M = M;
+    g.N = N;
+    g.K = K;
+    g.nb1 = 1;
+    return gemm_choice(g, b == 2 ? GEMM_B_CONV : b ? GEMM_B_NK : GEMM_B_KN, nb, aligned != 0,
+                       aligned != 0 && b != 2, o->ocl->cu_count);
+}
+
+extern "C" int icoreg_conv5_choice(struct ops *o, int nb, int C, int H, int W, int K, int pad)
+{
+    conv_args a = {};
+
+    a.C = C;
+    a.H = H;
+    a.W = W;
+    a.K = K;
+    a.pad = pad;
+    a.Ho = H + 2 * pad - 4;
+    a.Wo = W + 2 * pad - 4;
+    return conv_direct_choice(a, nb, o->ocl->cu_count);
+}
+
 /* ops_conv2d over nb images (in_stride / out_stride floats apart). */
 /* U: the filters already in Winograd form (conv_wino_prepare) or NULL. */
 static void conv_impl(struct ops *o, int nb, cl_mem in, long long in_stride,

@@ -86,6 +86,15 @@ void icoreg_conv_wino_form(int form);
  * stride 1, padding 1 convolution of nb contiguous C x H x W images to K
  * channels on o's device, under the current icoreg_conv_wino_form. */
 int icoreg_conv_wino_choice(struct ops *o, int nb, int C, int H, int W, int K);
+/* What the library runs on o's device (only its number of CUs matters):
+ * icoreg_gemm_choice, a product M x N x K of nb batches with B given K x N (b =
+ * 0), N x K (1) or gathered from a convolution's input (2), rows aligned to
+ * 16 bytes or not: 0 the fp32 matrix instructions, 1 the bf16 ones, 2 the bf16
+ * ones with tiles cut over K. icoreg_conv5_choice, a 5 x 5, stride 1
+ * convolution: 0 the fp32 instructions, else the bf16 ones with the input
+ * channels in that many pieces. For tests. */
+int icoreg_gemm_choice(struct ops *o, int M, int N, int K, int b, int nb, int aligned);
+int icoreg_conv5_choice(struct ops *o, int nb, int C, int H, int W, int K, int pad);
 /* How many times roma_match has re-run a GP solve through
  * roma_gp_solve_events after the in-kernel wait gave up. */
 int icoreg_roma_gp_retries(const struct roma_model *m);

@@ -1,11 +1,15 @@
 # SPDX-License-Identifier: Unlicense
 """GPU: 5 x 5 convolutions on the bf16 matrix instructions (at least 16
-channels in, 32 out and 96 blocks of 64 channels x 256 pixels) against
-torch's float64 convolution, at the edges of their blocks.
+channels in, 32 out and 96 blocks of 64 channels x 256 pixels, 256 with one
+chunk of input channels and more than 32 outputs) against torch's float64
+convolution, at the edges of their blocks. Each case asserts that it runs
+there (icoreg_conv5_choice).
 
 Bound: as for the products of tests/test_gemm_split_gpu.py, 2^-24 (n / 8 +
 16) sum |w x| over the n = 25 C terms, plus the input normalisation's
-rounding (three float32 steps a value, 3 * 2^-24 |w x|)."""
+rounding (three float32 steps a value, 3 * 2^-24 |w x|); for the rms error
+2^-24 sqrt((n / 8 + 16) / 3) of the output's rms, the normalisation's three
+steps and the bias's two."""
 
 import time
 
@@ -20,13 +24,22 @@ U = 2.0 ** -24
 # (images, C, K, H, W, pad, norm, act); act 0 none, 2 ReLU.
 CASES = [
     (1, 16, 32, 160, 160, 2, 1, 0),     # one slice of channels, half a block of outputs
-    (1, 17, 64, 161, 175, 2, 0, 2),     # a slice with one channel, ragged tiles
-    (1, 33, 65, 97, 190, 2, 1, 0),      # 64 channels and one on the few-channel kernel
+    (1, 17, 64, 240, 276, 2, 0, 2),     # a slice with one channel, ragged tiles
+    (1, 33, 65, 130, 190, 2, 1, 0),     # 64 channels and one on the few-channel kernel
     (2, 20, 150, 60, 127, 2, 1, 2),     # second block of 128 partly empty, pairs
     (1, 48, 128, 97, 130, 0, 0, 0),     # no padding, pieces over the channels
     (1, 100, 72, 113, 129, 4, 1, 0),    # padding past the window's half, pieces, K = 64 + 8
     (2, 40, 200, 67, 65, 1, 1, 2),
 ]
+# Sizes below those limits: the fp32 instructions.
+SMALL = [
+    (1, 17, 64, 161, 175, 2, 0, 2),
+    (1, 33, 65, 97, 190, 2, 1, 0),
+]
+
+
+def choice(dev, c):
+    return dev.api.icoreg_conv5_choice(dev.po, c[0], c[1], c[3], c[4], c[2], c[5])
 
 
 def tensors(c, seed):
@@ -64,23 +77,28 @@ def want(c, x, w, b, v):
     return (y.relu() if act else y).numpy(), size.numpy()
 
 
-@pytest.mark.parametrize("c", CASES, ids=[str(c) for c in CASES])
+@pytest.mark.parametrize("c", CASES + SMALL, ids=str)
 def test_edges(c, dev, ic):
-    print(f"[conv split] {c}", flush=True)
+    print(f"[conv split] {c} choice {choice(dev, c)}", flush=True)
+    assert (choice(dev, c) > 0) == (c in CASES)
     x, w, b, v = tensors(c, sum(c))
     got = run(dev, ic, c, x, w, b, v)
     ref, size = want(c, x, w, b, v)
     worst = np.max(np.abs(got - ref) / (U * (25 * c[1] / 8 + 19) * size))
-    print(f"[conv split] worst {worst:.3f} of the bound", flush=True)
+    rms = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    print(f"[conv split] worst {worst:.3f} of the bound, rms {rms:.2e}", flush=True)
     assert worst <= 1
+    if c in CASES:
+        assert rms <= U * (((25 * c[1] / 8 + 16) / 3) ** 0.5 + 5)
 
 
 def test_values_that_are_not_finite(dev, ic):
-    c = (1, 18, 40, 160, 165, 2, 0, 0)
+    c = (1, 18, 40, 240, 276, 2, 0, 0)
+    assert choice(dev, c) == 1
     x, w, b, _ = tensors(c, 5)
     x[0, 3, 0, 0] = np.inf
     x[0, 17, 80, 70] = np.nan
-    x[0, 0, 159, 164] = 3.4e38  # above the largest bf16
+    x[0, 0, 239, 275] = 3.4e38  # above the largest bf16
     w[7, 3, 2, 2] = 0           # inf * 0
     w[:, 0] *= 0.5              # no output overflows
     got = run(dev, ic, c, x, w, b, None)
@@ -104,6 +122,7 @@ def test_magnitudes(ex, ew, dev, ic):
     of the sum or more."""
     c = (1, 32, 40, 128, 200, 2, 0, 0)
     print(f"[conv split] magnitudes 2^{ex} 2^{ew}", flush=True)
+    assert choice(dev, c) == 2
     x, w, b, _ = tensors(c, 3)
     x = np.ldexp(x.astype(np.float64), ex).astype(np.float32)
     w = np.ldexp(w.astype(np.float64), ew).astype(np.float32)
@@ -124,6 +143,7 @@ def test_values_that_are_not_finite_again(c, dev, ic):
     filters, in the first and the last channels and at corners, come out as
     float32 products give them; outputs they do not reach are unmoved."""
     print(f"[conv split] not finite {c}", flush=True)
+    assert choice(dev, c) == (3 if c[1] == 36 else 1)
     x, w, b, v = tensors(c, 11)
     n, C, K, H, W, pad, norm, act = c
     x[0, 3, 0, 0] = np.inf
@@ -169,6 +189,7 @@ def test_cost_of_values_that_are_not_finite(dev, ic):
         return min(times)
 
     print("[conv split] cost", flush=True)
+    assert dev.api.icoreg_conv5_choice(dev.po, 1, C, H, W, K, 2) == 1
     clean, nan = best(1.0), best(np.nan)
     print(f"[conv split] {nan / clean:.2f} times", flush=True)
     assert np.isnan(dev.read(out)).all()

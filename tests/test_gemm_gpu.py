@@ -35,8 +35,9 @@ GEMM_SHAPES = [
     # Main kernel with tiles cut over K on 256 CUs (one batch, under 4
     # tiles per CU): 288 tiles (256 whole, 32 in 8 pieces) with in-place
     # residual and bias; 64 tiles in 4 pieces each, ragged edges, K not a
-    # multiple of 16.
+    # multiple of 16. The last, with K > 512, runs on the bf16 instructions.
     (1100, 1024, 512, 1, 1, 4, 1, 0),
+    (500, 500, 504, 1, 1, 1, 0, 1),
     (500, 500, 520, 1, 1, 1, 0, 1),
 ]
 

@@ -1,17 +1,25 @@
 # SPDX-License-Identifier: Unlicense
-"""GPU: ops_gemm on the bf16 matrix instructions (products of more than 512
-terms) against float64 sums, at the edges of its tiles and cuts.
+"""GPU: ops_gemm and the gathering convolution on the bf16 matrix
+instructions (products of more than 512 terms, but for small grids) against
+float64 sums, at the edges of their tiles and cuts. Each case states which
+instructions it is for (icoreg_gemm_choice).
 
 Bound: a value's six kept bf16 products leave out less than 2^-25 of |a b|;
 the matrix core adds groups of eight k, so K / 8 additions round by 2^-24 of
 a partial sum that sum |a b| bounds, and a group's alignment drops at most
 8 * 2^-24 of its largest product: 2^-24 (K / 8 + 16) sum |a b| in all, and
-the float32 epilogue's own 2^-24 a step."""
+the float32 epilogue's own 2^-24 a step. That worst case would hide a lost
+part, so the rms error is bounded too: of random sign, K / 8 + 16 roundings
+of partial sums whose rms is at most the sum's make 2^-24 sqrt((K / 8 + 16) /
+3) of it, and the epilogue two more. (The products hl and lh left out make
+2^-19 or more.)"""
 
 import time
 
 import numpy as np
 import pytest
+import torch
+import torch.nn.functional as F
 
 pytestmark = pytest.mark.gpu
 
@@ -19,24 +27,43 @@ U = 2.0 ** -24
 
 # (M, N, K, transb, nb, act, residual, biasrow); act 0 none, 2 ReLU, 3 leaky.
 SHAPES = [
-    # One output, one row, one column; K just past the rule, K % 32 != 0.
-    (1, 1, 513, 1, 1, 0, 0, 0),
-    (1, 70, 516, 0, 1, 0, 1, 1),
-    (70, 1, 544, 1, 1, 3, 0, 0),
-    # Around one and two 64- and 128-row tiles, aligned and not.
-    (64, 64, 544, 1, 1, 0, 0, 0),
-    (65, 63, 1023, 1, 1, 2, 0, 1),
-    (128, 128, 576, 0, 2, 0, 1, 0),
-    (129, 127, 577, 0, 1, 3, 0, 1),
+    # One output, one row, one column; K % 32 != 0.
+    (1, 1, 1028, 1, 1, 0, 0, 0),
+    (1, 72, 1032, 0, 1, 0, 1, 1),
+    (70, 1, 1056, 1, 1, 3, 0, 0),
+    # Around one and two 64-row tiles.
+    (64, 64, 1056, 1, 1, 0, 0, 0),
+    (65, 63, 1028, 1, 1, 2, 0, 1),
+    (63, 64, 1060, 0, 1, 0, 1, 0),
+    (128, 128, 1056, 0, 2, 0, 1, 0),
+    (129, 128, 1060, 0, 1, 3, 0, 1),
+    (129, 127, 1060, 1, 1, 3, 0, 1),
     (127, 260, 1140, 0, 3, 2, 1, 0),
+    # K just past the rule, 49 tiles of 64 x 64.
+    (448, 448, 516, 1, 1, 0, 1, 0),
+    (448, 448, 516, 0, 1, 3, 0, 1),
     # Every tile cut over K (few tiles, long K); the last piece shorter.
     (100, 90, 4100, 1, 1, 0, 1, 0),
     (96, 200, 2052, 0, 1, 3, 0, 1),
     # No 16-byte loads: 99 and 121 tiles of 64 x 64 (fewer run elsewhere).
     (700, 520, 577, 1, 1, 2, 1, 0),
     (650, 701, 1023, 0, 1, 0, 0, 1),
+    # 64 x 128 tiles.
+    (150, 5348, 532, 1, 4, 3, 1, 0),
+    (152, 5056, 576, 0, 4, 0, 0, 1),
     # 288 tiles of 128 x 128: 256 whole, 32 cut.
     (2304, 2000, 1024, 1, 1, 0, 1, 0),
+]
+# Sums of more than 512 terms outside the rule: few tiles, no 16-byte loads or
+# under 1024 terms (fp32 instructions).
+SMALL = [
+    (1, 1, 513, 1, 1, 0, 0, 0),
+    (1, 70, 516, 0, 1, 0, 1, 1),
+    (70, 1, 544, 1, 1, 3, 0, 0),
+    (64, 64, 544, 1, 1, 0, 0, 0),
+    (65, 63, 1023, 1, 1, 2, 0, 1),
+    (128, 128, 576, 0, 2, 0, 1, 0),
+    (129, 127, 577, 0, 1, 3, 0, 1),
 ]
 
 
@@ -51,10 +78,12 @@ def run(dev, ic, a, b, shape, alpha, bias, r):
     return dev.read(out, nb * M * N).reshape(nb, M, N)
 
 
-@pytest.mark.parametrize("shape", SHAPES, ids=[str(s) for s in SHAPES])
+@pytest.mark.parametrize("shape", SHAPES + SMALL, ids=str)
 def test_edges(shape, dev, ic):
     M, N, K, transb, nb, act, residual, biasrow = shape
-    print(f"[gemm split] {shape}", flush=True)
+    choice = dev.api.icoreg_gemm_choice(dev.po, M, N, K, transb, nb, 1)
+    print(f"[gemm split] {shape} choice {choice}", flush=True)
+    assert (choice > 0) == (shape in SHAPES)
     rng = np.random.default_rng(M + 3 * N + K)
     a = rng.standard_normal((nb, M, K)).astype(np.float32)
     b = rng.standard_normal((nb, N, K) if transb else (nb, K, N)).astype(np.float32)
@@ -70,8 +99,11 @@ def test_edges(shape, dev, ic):
         v += r
     size = 0.5 * (np.abs(a).astype(np.float64) @ np.abs(bt).astype(np.float64)) + 2
     worst = np.max(np.abs(got - v) / (U * ((K / 8 + 16) * size + 4 * np.abs(v))))
-    print(f"[gemm split] worst {worst:.3f} of the bound", flush=True)
+    rms = np.linalg.norm(got - v) / np.linalg.norm(v)
+    print(f"[gemm split] worst {worst:.3f} of the bound, rms {rms:.2e}", flush=True)
     assert worst <= 1
+    if choice and M * N >= 64:
+        assert rms <= U * (((K / 8 + 16) / 3) ** 0.5 + 2)
 
 
 @pytest.mark.parametrize("transb", [0, 1])
@@ -170,3 +202,73 @@ def test_cost_of_values_that_are_not_finite(transb, dev, ic):
     print(f"[gemm split] {nan / clean:.2f} times", flush=True)
     assert np.isnan(dev.read(out, M * N)).all()
     assert nan <= 4 * clean
+
+
+# (images, C, K, H, W, window, pad, dilation, stride, norm): more than 512
+# terms in shapes that neither the direct nor the Winograd kernels take.
+CONVS = [
+    (1, 11, 24, 30, 33, 7, 3, 1, 1, 0),    # 539 terms: no 16-byte loads of the filters
+    (1, 12, 40, 37, 29, 7, 2, 1, 1, 1),    # 588
+    (2, 64, 65, 20, 21, 3, 2, 2, 1, 1),    # dilated, pairs, 576
+    (1, 72, 130, 40, 40, 3, 1, 2, 2, 0),
+    (1, 3, 70, 112, 84, 14, 0, 1, 14, 0),  # patches, 588
+    (1, 130, 200, 64, 70, 3, 2, 2, 1, 1),
+]
+
+
+def conv(dev, ic, c, x, w, b, v):
+    n, C, K, H, W, k, pad, dil, stride, norm = c
+    ho, wo = ((s + 2 * pad - dil * (k - 1) - 1) // stride + 1 for s in (H, W))
+    X, Wt, B, out = dev.upload(x), dev.upload(w), dev.upload(b), dev.zeros(n * K * ho * wo)
+    V = [dev.upload(t) for t in v] if norm else [None] * 3
+    g = ic.geom(k, k, stride, stride, pad, pad, dil, dil, 1)
+    dev.api.ops_conv2d_batch(dev.po, n, X.mem, C * H * W, C, H, W, Wt.mem, B.mem, K, ic.C.byref(g),
+                             *(ic.mem(t) for t in V), 0, 0.0, out.mem, K * ho * wo)
+    return dev.read(out).reshape(n, K, ho, wo)
+
+
+@pytest.mark.parametrize("finite", [1, 0])
+@pytest.mark.parametrize("c", CONVS, ids=str)
+def test_gathered_convolution(c, finite, dev, ic):
+    """The input normalised and gated while it is gathered, padding 0; with
+    an infinity, a NaN and a value without a split the sums they reach come
+    out as float32 products give them (each of K terms rounds)."""
+    n, C, K, H, W, k, pad, dil, stride, norm = c
+    ho, wo = ((s + 2 * pad - dil * (k - 1) - 1) // stride + 1 for s in (H, W))
+    terms = C * k * k
+    print(f"[gemm split] conv {c} finite {finite}", flush=True)
+    assert dev.api.icoreg_gemm_choice(dev.po, K, ho * wo, terms, 2, n, 1) == 1
+    rng = np.random.default_rng(sum(c))
+    x = rng.standard_normal((n, C, H, W)).astype(np.float32)
+    w = (rng.standard_normal((K, C, k, k)) / terms ** 0.5).astype(np.float32)
+    b = rng.uniform(-0.1, 0.1, K).astype(np.float32)
+    v = [rng.uniform(lo, hi, C).astype(np.float32) for lo, hi in ((-0.2, 0.2), (0.8, 1.25), (0.1, 0.3))]
+    if not finite:
+        x[0, 2, 1, 1] = np.inf  # odd places: the strided case reads no other
+        x[n - 1, C - 1, H // 4 * 2 + 1, W // 4 * 2 + 1] = np.nan
+        x[0, 0, 3, W // 2 * 2 - 5] = 2e38  # above 2^104
+        w[3, 2] = 0               # inf * 0
+        w[:, 0] *= 0.25           # no output overflows
+    got = conv(dev, ic, c, x, w, b, v)
+    t = torch.from_numpy(x).double()
+    if norm:
+        m, r, a = (torch.from_numpy(q).double()[:, None, None] for q in v)
+        t = (t - m) * r
+        t = torch.where(t >= 0, t, a * t)
+    args = {"padding": pad, "dilation": dil, "stride": stride}
+    wd, bd = torch.from_numpy(w).double(), torch.from_numpy(b).double()
+    want = F.conv2d(t, wd, bd, **args).numpy()
+    size = F.conv2d(t.abs(), wd.abs(), bd.abs(), **args).numpy()
+    if finite:
+        worst = np.max(np.abs(got - want) / (U * (terms / 8 + 19) * size))
+        rms = np.linalg.norm(got - want) / np.linalg.norm(want)
+        print(f"[gemm split] worst {worst:.3f} of the bound, rms {rms:.2e}", flush=True)
+        assert worst <= 1 and rms <= U * (((terms / 8 + 16) / 3) ** 0.5 + 5)
+        return
+    with np.errstate(over="ignore"):
+        want32 = want.astype(np.float32)
+    assert np.array_equal(np.isnan(got), np.isnan(want32))
+    assert np.array_equal(got[np.isinf(want32)], want32[np.isinf(want32)])
+    fine = np.isfinite(want32)
+    assert fine.any() and not fine.all()
+    assert np.max(np.abs(got[fine] - want[fine]) / (U * (terms + 19) * size[fine])) <= 1
