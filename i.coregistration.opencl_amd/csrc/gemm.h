@@ -74,7 +74,7 @@ size_t gemm_part_floats(const gemm_args &g, int bmode, int nb, bool va, bool vb,
  * instructions (gemm_split.hip). */
 void gemm_split_launch(const gemm_args &g, int bmode, int nb, bool va, bool vb, int cus,
                        hipStream_t s);
-size_t gemm_split_floats(const gemm_args &g, int bmode, int nb, int cus);
+size_t gemm_split_floats(const gemm_args &g, int bmode, int nb, bool va, bool vb, int cus);
 
 /* What gemm_launch runs a product of g's M, N, K on: 0 the fp32
  * instructions, 1 the bf16 ones, 2 the bf16 ones with tiles cut over K. */

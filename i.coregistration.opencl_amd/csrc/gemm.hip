@@ -1,8 +1,8 @@
 /* SPDX-License-Identifier: Unlicense */
 
 /* fp32 GEMM on the CDNA4 fp32 matrix instructions: C = act(alpha A op(B) +
- * bias) + R. Products of K up to GEMM_SPLIT_K (gemm_launch); longer ones run
- * in gemm_split.hip.
+ * bias) + R. Products of K up to GEMM_SPLIT_K, and longer ones of small
+ * grids (gemm_split_ok); the others run in gemm_split.hip.
  *
  * The contract is the reference's gemm / gemm_big (ops.cl:39-284 of
  * i.coregistration.opencl): batched over nb = nb0 * nb1 with two batch
@@ -914,19 +914,24 @@ static bool gemm_plan(const gemm_args &g, int bmode, int nb, int cus, int &nfull
 }
 
 /* Products that run on the bf16 instructions (gemm_split.hip): sums of
- * more than GEMM_SPLIT_K products. Alone the shorter ones gain too, most of
- * them under a fifth (ELoFTR's K = 128 .. 512: 1.14 -> 1.04 ms a pair), but
- * the bf16 instructions draw more power than the fp32 ones and the kernels
- * around them then run at a lower clock (ELoFTR's fp32 convolutions 8 - 10 %
- * slower: 4.12 -> 4.23 ms a pair in all). */
+ * more than GEMM_SPLIT_K products. Alone the shorter ones gain too (6400 x
+ * 256 x 256 20.1 -> 13.5 us, 3200 x 1024 x 512 38 -> 31), but the bf16
+ * instructions draw more power than the fp32 ones, and the kernels around
+ * them then run at a lower clock: ELoFTR, whose products are those, took 4.24 ms
+ * a pair in all with a limit of 128 against 4.19. */
 #define GEMM_SPLIT_K 512
 
 /* Where 64 x 64 tiles are few, a block's time is its loads, and splitting
- * while staging adds to it: without 16-byte loads below 3 / 8 of the CUs
- * (148 x 685 x 512 10.2 us against 13.7, 24 x 683 x 1024 9.6 against 12.4, 318
- * x 675 x 535 13.2 against 14.3; 2896 x 2893 x 3175 1089 -> 514), with them below 1024
- * products and 48 tiles (397 x 872 x 256 9.9 against 10.4; 398 x 868 x 1379
- * 23.5 -> 19.1). va, vb: 16-byte loads of A and B. */
+ * while staging adds to it: with 16-byte loads below 48 tiles and 1024
+ * products (192 x 320 x 768 8.5 us against 9.3, 384 x 448 x 1020 11.6 against
+ * 12.4; M x N x K, B given N x K), without them below 3 / 8 of the CUs (300 x 500
+ * x 769 13.7 against 14.8). On the other side of these lines 4254 products (M, N
+ * 16 .. 4096, K to 4096) took 0.75 of the fp32 kernels' time at the mean, one
+ * in 27 more than 1.05 of it, none more than 1.2 (few tiles, K 1028 .. 1500: 128
+ * x 256 x 1028 9.9 us against 9.1); they stay there for their smaller error. A
+ * gathered convolution is always faster (64 -> 64 channels, 7 x 7 at 14 x 14 353
+ * -> 198 us, 64 -> 32 channels, 3 x 3 dilated at 8 x 8 51 -> 40).
+ * va, vb: 16-byte loads of A and B. */
 static bool gemm_split_ok(const gemm_args &g, int bmode, int nb, bool va, bool vb, int cus)
 {
     const long long tiles = (long long)nb * ((g.M + 63) / 64) * ((g.N + 63) / 64);
@@ -943,7 +948,7 @@ int gemm_choice(const gemm_args &g, int bmode, int nb, bool va, bool vb, int cus
     va = va && g.K % 4 == 0;
     vb = vb && (bmode == GEMM_B_KN ? g.N % 4 == 0 : g.K % 4 == 0);
     return !gemm_split_ok(g, bmode, nb, va, vb, cus)     ? 0
-           : gemm_split_floats(g, bmode, nb, cus) == 0 ? 1
+           : gemm_split_floats(g, bmode, nb, va, vb, cus) == 0 ? 1
                                                          : 2;
 }
 
@@ -955,7 +960,7 @@ size_t gemm_part_floats(const gemm_args &g, int bmode, int nb, bool va, bool vb,
     va = va && g.K % 4 == 0;
     vb = vb && (bmode == GEMM_B_KN ? g.N % 4 == 0 : g.K % 4 == 0);
     if (bf16 && gemm_split_ok(g, bmode, nb, va, vb, cus))
-        return gemm_split_floats(g, bmode, nb, cus);
+        return gemm_split_floats(g, bmode, nb, va, vb, cus);
     if (gemm_smallk_ok(g, bmode, nb, va, vb, cus) || gemm_dma_ok(g, bmode, va, vb) ||
         !gemm_plan(g, bmode, nb, cus, nfull, split))
         return 0;

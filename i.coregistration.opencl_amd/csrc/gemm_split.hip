@@ -467,58 +467,76 @@ long long split_tiles(int tile, int M, int N)
            ((N + split_bn[tile] - 1) / split_bn[tile]);
 }
 
-/* The tile shape and cut with the smallest estimated time on cus CUs: that
- * of the CU with the most tiles. n tiles of a CU take n * share us a 1024
- * of K, but no less than alone (one tile's waves do not fill the CU), and
- * n * fixed us for their ends (figures from sweeps of ViT, refiner and
- * ELoFTR shapes; split_m alone runs as fast as two together, so equal
- * shares decide). With one batch and a plain epilogue, the tiles left over
- * after an equal whole number a CU, or all of them, may be cut over K into
- * up to SPLIT_MAX pieces of at least 128 k, for the pieces' sums written
- * and read (at about 4.5 TB/s) and a second launch. */
-split_choice split_plan(int M, int N, int K, int nb, bool cut, int cus)
+/* Time model of a tile shape's grid, us: a CU's m tiles take m share a 1024 of
+ * K, but no less than alone (one tile's waves do not fill the CU), and m fixed
+ * for their ends; call for the launch and a tile's first loads, cut for the
+ * second launch where tiles are cut over K. */
+struct split_cost {
+    double alone, share, fixed, call, cut;
+};
+
+/* split_m, split_s and split_xs by how the operands come (split_row), fitted to 170000 times of 11600 products (M, N 16 .. 4096, K 513 .. 4096, every
+ * tile and cut) on an MI355X: 16-byte rows within 2 - 3 % of them at the
+ * median, 4-byte loads within 4 - 8 %. The gathered convolution, which is never
+ * cut, has figures from the patch embedding. */
+const split_cost split_costs[5][3] = {
+    /* B N x K, 16-byte rows; else */
+    {{41.6, 30.3, 1.6, 6.3, 0.0}, {35.1, 21.8, 0.1, 7.4, 0.0}, {22.5, 13.6, 0.0, 6.3, 0.8}},
+    {{93.4, 76.0, 0.0, 0.0, 5.1}, {73.4, 55.1, 0.0, 6.7, 0.0}, {50.7, 38.3, 0.0, 3.9, 2.2}},
+    /* B K x N, 16-byte rows of A; else */
+    {{48.7, 34.4, 0.9, 7.1, 0.0}, {47.7, 26.2, 0.2, 7.5, 0.0}, {29.7, 14.3, 0.0, 6.4, 0.9}},
+    {{74.8, 45.5, 4.7, 0.0, 1.6}, {62.9, 35.5, 0.0, 6.9, 0.1}, {44.9, 25.2, 0.0, 4.9, 1.6}},
+    /* B gathered */
+    {{42.0, 42.0, 4.0, 0.0, 0.0}, {35.0, 23.0, 2.5, 0.0, 0.0}, {22.0, 13.0, 1.0, 0.0, 0.0}},
+};
+
+int split_row(int bmode, bool va, bool vb)
 {
-    static const struct {
-        double share, alone, fixed;
-    } cost[3] = {{42.0, 42.0, 4.0}, {23.0, 35.0, 2.5}, {13.0, 22.0, 1.0}};
+    return bmode == GEMM_B_NK ? (va && vb ? 0 : 1) : bmode == GEMM_B_KN ? (va ? 2 : 3) : 4;
+}
+
+/* The tile shape and cut with the smallest estimated time on cus CUs. With
+ * one batch and a plain epilogue, the tiles left over after an equal whole
+ * number a CU, or all of them, may be cut over K into up to SPLIT_MAX pieces
+ * of at least 128 k. */
+split_choice split_plan(const gemm_args &g, int row, int nb, bool cut, int cus)
+{
     split_choice best = {2, 0, 1};
     double tbest = 1e30;
+    const double k = std::max(g.K, 32) / 1024.0;
+    /* whole tiles, and pieces of 1 / s of K (their sums written and read at
+     * about 4.5 TB/s): the CU with the most, past four of them leveled out. */
+    auto consider = [&](int i, int full, long long whole, int pieces, int s) {
+        const split_cost &c = split_costs[row][i];
+        auto part = [&](long long n, int pieces_) {
+            const double m =
+                n <= 4LL * cus ? (double)((n + cus - 1) / cus) : (double)n / cus + 0.5;
+
+            return n ? std::max(c.alone, m * c.share) * k / pieces_ + m * c.fixed : 0.0;
+        };
+        double t = c.call + part(whole, 1);
+
+        if (pieces)
+            t += part(pieces, s) + c.cut + 8.0 * pieces * split_bm[i] * split_bn[i] / 4.5e6;
+        if (t < tbest) {
+            tbest = t;
+            best = {i, full, s};
+        }
+    };
 
     for (int i = 0; i < 3; i++) {
-        const long long n = split_tiles(i, M, N), units = n * nb;
-        const double k = std::max(K, 32) / 1024.0;
-        /* m tiles of 1 / s of K on one CU, past four of them leveled out. */
-        auto time = [&](double units_, int s) {
-            const double m = units_ <= 4.0 * cus ? (double)(((long long)units_ + cus - 1) / cus)
-                                                 : units_ / cus + 0.5;
+        const long long n = split_tiles(i, g.M, g.N);
 
-            return m > 0 ? std::max(cost[i].alone, m * cost[i].share) * k / s + m * cost[i].fixed
-                         : 0.0;
-        };
-        const double t1 = time((double)units, 1);
-
-        if (t1 < tbest) {
-            tbest = t1;
-            best = {i, 0, 1};
-        }
+        consider(i, 0, n * nb, 0, 1);
         if (!cut || nb != 1 || n >= 4LL * cus)
             continue;
-        const int rem = (int)(n % cus), smax = std::min(K / 128, SPLIT_MAX);
+        const int all = (int)n, rem = all % cus, smax = std::min(g.K / 128, SPLIT_MAX);
 
-        for (int s = 2; s <= smax; s++)
-            for (int all = 0; all < 2; all++) {
-                const int tail = all ? (int)n : rem, full = (int)n - tail;
-
-                if (tail == 0 || (!all && full == 0))
-                    continue;
-                const double bytes = 8.0 * tail * s * split_bm[i] * split_bn[i];
-                const double t = time(full, 1) + time((double)tail * s, s) + bytes / 4.5e6 + 4.0;
-
-                if (t < tbest) {
-                    tbest = t;
-                    best = {i, full, s};
-                }
-            }
+        for (int s = 2; s <= smax; s++) {
+            consider(i, 0, 0, all * s, s);
+            if (rem && rem < all)
+                consider(i, all - rem, all - rem, rem * s, s);
+        }
     }
     return best;
 }
@@ -557,11 +575,11 @@ bool split_cut_ok(const gemm_args &g, int bmode, int nb)
 
 } // namespace
 
-size_t gemm_split_floats(const gemm_args &g, int bmode, int nb, int cus)
+size_t gemm_split_floats(const gemm_args &g, int bmode, int nb, bool va, bool vb, int cus)
 {
     if (!split_cut_ok(g, bmode, nb))
         return 0;
-    const split_choice c = split_plan(g.M, g.N, g.K, nb, true, cus);
+    const split_choice c = split_plan(g, split_row(bmode, va, vb), nb, true, cus);
 
     return c.split > 1 ? (size_t)(split_tiles(c.tile, g.M, g.N) - c.nfull) * c.split *
                              split_bm[c.tile] * split_bn[c.tile]
@@ -571,8 +589,8 @@ size_t gemm_split_floats(const gemm_args &g, int bmode, int nb, int cus)
 void gemm_split_launch(const gemm_args &g, int bmode, int nb, bool va, bool vb, int cus,
                        hipStream_t s)
 {
-    const split_choice c =
-        split_plan(g.M, g.N, g.K, nb, g.part && split_cut_ok(g, bmode, nb), cus);
+    const split_choice c = split_plan(g, split_row(bmode, va, vb), nb,
+                                      g.part && split_cut_ok(g, bmode, nb), cus);
     gemm_args a = g;
 
     a.nfull = c.nfull;

@@ -151,3 +151,15 @@ def test_roma_kernels_reject_bad_sizes(ic):
             api.roma_dwpw_small(C.byref(ops), b, 8, 4, 4, a, a, a, a, a)
         lib.ocl_release(C.byref(b))
     lib.ocl_release(C.byref(a))
+
+
+def test_long_products_are_cut_where_cus_would_wait(ic):
+    """A grid of at most one tile a CU leaves a CU its tile's whole sum; what
+    rows without 16-byte loads cost a tile makes cutting it over K pay, also
+    just past 512 terms (961 x 466 x 526 whole 30 us, cut 20)."""
+    b, o = ic.OclBackend(cu_count=256), ic.Ops()
+    o.ocl = C.pointer(b)
+    for M, N, K, transb, aligned in ((961, 466, 526, 1, 0), (1243, 814, 837, 1, 0),
+                                     (893, 792, 867, 0, 0), (768, 640, 516, 1, 1),
+                                     (144, 3928, 808, 0, 1)):
+        assert ic.lib().icoreg_gemm_choice(C.byref(o), M, N, K, transb, 1, aligned) == 2, (M, N, K)
