@@ -43,10 +43,11 @@
 #define GEMM_MAX_SPLIT 8
 
 /* BM x BN output tile, BK slice, WGM x WGN waves (each a
- * BM / WGM x BN / WGN block of 32 x 32 MFMA tiles). */
-template <int BM, int BN, int BK, int MODE, bool VA, bool VB, int WGM = 2,
+ * BM / WGM x BN / WGN block of 32 x 32 MFMA tiles), registers for OCC waves a
+ * SIMD (launch_cfg). */
+template <int BM, int BN, int BK, int OCC, int MODE, bool VA, bool VB, int WGM = 2,
           int WGN = 2>
-__global__ void __launch_bounds__(64 * WGM * WGN) gemm_mfma(const gemm_args g)
+__global__ void __launch_bounds__(64 * WGM * WGN, OCC) gemm_mfma(const gemm_args g)
 {
     constexpr int NTH = 64 * WGM * WGN;
     constexpr int LDSA = BM + GEMM_PAD, LDSB = BN + GEMM_PAD;
@@ -771,7 +772,7 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_dma(const gemm_args g)
     gemm_epilogue<TM, TN>(g, acc, b0, b1, m0 + wm * (BM / WM), n0 + wn * (BN / WN), lane);
 }
 
-template <int BM, int BN, int BK, int WGM, int WGN, int MODE>
+template <int BM, int BN, int BK, int OCC, int WGM, int WGN, int MODE>
 static void launch_mode(const gemm_args &g, int nb, bool va, bool vb,
                         hipStream_t s, int blocks)
 {
@@ -779,7 +780,7 @@ static void launch_mode(const gemm_args &g, int nb, bool va, bool vb,
     dim3 grid(blocks > 0 ? blocks : tiles, nb), block(64 * WGM * WGN);
 
 #define GEMM_LAUNCH(VA_, VB_)                                                  \
-    hipLaunchKernelGGL((gemm_mfma<BM, BN, BK, MODE, VA_, VB_, WGM, WGN>),      \
+    hipLaunchKernelGGL((gemm_mfma<BM, BN, BK, OCC, MODE, VA_, VB_, WGM, WGN>), \
                        grid, block, 0, s, g)
     if (MODE == GEMM_B_CONV) {
         if (va)
@@ -798,21 +799,38 @@ static void launch_mode(const gemm_args &g, int nb, bool va, bool vb,
 #undef GEMM_LAUNCH
 }
 
-template <int BM, int BN, int BK, int WGM, int WGN>
-static void launch_cfg(const gemm_args &g, int bmode, int nb, bool va,
+template <int BM, int BN, int BK, int OCC, int WGM, int WGN>
+static void launch_occ(const gemm_args &g, int bmode, int nb, bool va,
                        bool vb, hipStream_t s, int blocks)
 {
     switch (bmode) {
     case GEMM_B_KN:
-        launch_mode<BM, BN, BK, WGM, WGN, GEMM_B_KN>(g, nb, va, vb, s, blocks);
+        launch_mode<BM, BN, BK, OCC, WGM, WGN, GEMM_B_KN>(g, nb, va, vb, s, blocks);
         break;
     case GEMM_B_NK:
-        launch_mode<BM, BN, BK, WGM, WGN, GEMM_B_NK>(g, nb, va, vb, s, blocks);
+        launch_mode<BM, BN, BK, OCC, WGM, WGN, GEMM_B_NK>(g, nb, va, vb, s, blocks);
         break;
     default:
-        launch_mode<BM, BN, BK, WGM, WGN, GEMM_B_CONV>(g, nb, va, vb, s, blocks);
+        launch_mode<BM, BN, BK, OCC, WGM, WGN, GEMM_B_CONV>(g, nb, va, vb, s, blocks);
         break;
     }
+}
+
+/* The epilogue loads half a tile's bias and residual at once, for which the
+ * kernel left to itself takes the registers of 5 waves a SIMD. Grids of many
+ * tiles a CU live on the waves: from 8 on, with registers for 7, 12800 x 1024 x
+ * 384 92.5 -> 90.3 us. Smaller ones gain too alone (3200 x 1024 x 512 38.2 -> 37.1),
+ * but not between ELoFTR's convolutions (4.17 -> 4.19 ms a pair). */
+template <int BM, int BN, int BK, int WGM, int WGN>
+static void launch_cfg(const gemm_args &g, int bmode, int nb, bool va, bool vb, int cus,
+                       hipStream_t s, int blocks)
+{
+    const long long tiles = (long long)((g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN) * nb;
+
+    if (tiles >= 8LL * cus)
+        launch_occ<BM, BN, BK, 7, WGM, WGN>(g, bmode, nb, va, vb, s, blocks);
+    else
+        launch_occ<BM, BN, BK, 5, WGM, WGN>(g, bmode, nb, va, vb, s, blocks);
 }
 
 bool gemm_shape_ok(const gemm_args &g, int bmode)
@@ -1028,11 +1046,11 @@ void gemm_launch(const gemm_args &g, int bmode, int nb, bool va, bool vb,
 
             gs.nfull = nfull;
             gs.split = split;
-            launch_cfg<64, 64, 16, 2, 2>(gs, bmode, nb, va, vb, s, nfull + (int)tail * split);
+            launch_cfg<64, 64, 16, 2, 2>(gs, bmode, nb, va, vb, cus, s, nfull + (int)tail * split);
             hipLaunchKernelGGL(gemm_pieces_kernel, dim3((unsigned)((tail * 4096 + 255) / 256)),
                                dim3(256), 0, s, gs, (int)tail);
             return;
         }
     }
-    launch_cfg<64, 64, 16, 2, 2>(g, bmode, nb, va, vb, s, 0);
+    launch_cfg<64, 64, 16, 2, 2>(g, bmode, nb, va, vb, cus, s, 0);
 }
