@@ -435,15 +435,32 @@ conv_split_plan conv_split_choose(const conv_args &a, int ks, int st, int nb, in
     const long long blocks = tiles(p.tw) * ((a.K + p.bm - 1) / p.bm) * nb;
     const int nc = (a.C + 15) / 16;
 
-    /* Fewer blocks than CUs: pieces over the input channels, about two
-     * blocks a CU, none empty. */
-    p.split = 1;
-    if (blocks < cus) {
-        int s = (int)std::min((2LL * cus + blocks - 1) / blocks, (long long)std::min(nc, 16));
-        const int per = (nc + s - 1) / s;
+    /* Pieces over the input channels where they shorten the slowest CU's
+     * share. A CU holds one block (its LDS), and a round of blocks takes about 9
+     * us and a slice of 16 channels 14.4 us (64 output channels) or 20.8 (128),
+     * 2.5 and 1.4 more where it is normalised; pieces write and read their sums
+     * at 2.3 or 3.6 TB/s (fitted to 22000 times of 7100 layers, within 5 % at the
+     * median). Cut into about two blocks a CU instead, one layer in two ran 5 %
+     * or more longer than it could, up to 1.6 times, and one in eight longer
+     * than on conv_mfma, up to 1.9 times (19 -> 256 channels, normalised, at 38 x
+     * 470: 83 us there, 97 in two pieces, 72 whole); so cut, one in 20, layers of 17
+     * to 21 channels whose second slice is nearly empty, up to 1.4 times. */
+    const double slice = p.bm == 64 ? 14.4 + (a.mean ? 2.5 : 0.0) : 20.8 + (a.mean ? 1.4 : 0.0);
+    const double mb = 8e-6 * nb * a.K * a.Ho * a.Wo / (p.bm == 64 ? 2.3 : 3.6);
+    double best = 1e30;
 
-        s = (nc + per - 1) / per;
-        p.split = nb * (long long)s > 65535 ? 1 : s;
+    p.split = 1;
+    for (int s = 1; s <= std::min(nc, 16); s++) {
+        const int per = (nc + s - 1) / s;
+        const long long n = blocks * s;
+        const double rounds = n <= 4LL * cus ? (double)((n + cus - 1) / cus) : (double)n / cus + 0.5;
+        const double us = rounds * (8.6 + slice * per) + (s > 1 ? mb * s : 0.0);
+
+        /* None empty, and the pieces' grid in range. */
+        if ((nc + per - 1) / per == s && (s == 1 || nb * (long long)s <= 65535) && us < best) {
+            best = us;
+            p.split = s;
+        }
     }
     /* Below 96 blocks of 64 channels on 256 CUs the smaller blocks of
      * conv_mfma win (128 -> 64 channels at 128 x 128, 64 blocks: 79 us against

@@ -91,8 +91,8 @@ int icoreg_conv_wino_choice(struct ops *o, int nb, int C, int H, int W, int K);
  * 0), N x K (1) or gathered from a convolution's input (2), rows aligned to
  * 16 bytes or not: 0 the fp32 matrix instructions, 1 the bf16 ones, 2 the bf16
  * ones with tiles cut over K. icoreg_conv5_choice, a 5 x 5, stride 1
- * convolution: 0 the fp32 instructions, else the bf16 ones with the input
- * channels in that many pieces. For tests. */
+ * convolution without normalisation: 0 the fp32 instructions, else the bf16
+ * ones with the input channels in that many pieces. For tests. */
 int icoreg_gemm_choice(struct ops *o, int M, int N, int K, int b, int nb, int aligned);
 int icoreg_conv5_choice(struct ops *o, int nb, int C, int H, int W, int K, int pad);
 /* How many times roma_match has re-run a GP solve through

@@ -163,3 +163,14 @@ def test_long_products_are_cut_where_cus_would_wait(ic):
                                      (893, 792, 867, 0, 0), (768, 640, 516, 1, 1),
                                      (144, 3928, 808, 0, 1)):
         assert ic.lib().icoreg_gemm_choice(C.byref(o), M, N, K, transb, 1, aligned) == 2, (M, N, K)
+
+
+def test_convolutions_are_cut_where_a_round_of_blocks_gets_shorter(ic):
+    """A CU holds one block of the bf16 5 x 5 convolution: 150 blocks run as one
+    round, in two pieces as two; 63 have room for four pieces."""
+    b, o = ic.OclBackend(cu_count=256), ic.Ops()
+    o.ocl = C.pointer(b)
+    for n, c, h, w, k, pieces in ((1, 19, 38, 470, 256, 1), (2, 42, 39, 261, 193, 1),
+                                  (1, 39, 128, 461, 36, 1), (1, 64, 97, 130, 128, 4),
+                                  (1, 80, 512, 512, 129, 1)):
+        assert ic.lib().icoreg_conv5_choice(C.byref(o), n, c, h, w, k, 2) == pieces, (n, c, h, w, k)

@@ -134,7 +134,7 @@ def test_magnitudes(ex, ew, dev, ic):
     assert rms <= U * ((25 * c[1] / 8 + 16) / 3) ** 0.5
 
 
-# Pieces over three slices of channels; normalised, 128 outputs a block, 16
+# Three slices of channels in two pieces; normalised, 128 outputs a block, 16
 # and 32 pixels wide tiles.
 @pytest.mark.parametrize("c", [(1, 36, 40, 160, 165, 2, 0, 0), (1, 33, 128, 200, 330, 2, 1, 0),
                                (1, 34, 200, 120, 384, 1, 1, 0)], ids=str)
@@ -143,7 +143,7 @@ def test_values_that_are_not_finite_again(c, dev, ic):
     filters, in the first and the last channels and at corners, come out as
     float32 products give them; outputs they do not reach are unmoved."""
     print(f"[conv split] not finite {c}", flush=True)
-    assert choice(dev, c) == (3 if c[1] == 36 else 1)
+    assert choice(dev, c) == (2 if c[1] == 36 else 1)
     x, w, b, v = tensors(c, 11)
     n, C, K, H, W, pad, norm, act = c
     x[0, 3, 0, 0] = np.inf
