@@ -40,8 +40,8 @@ ROOT = Path(__file__).resolve().parent
 PKG_DIR = ROOT / "i.coregistration.opencl_amd"
 PEAK_FP32_MFMA = 157.3  # TFLOP/s, MI355X dense fp32 matrix
 # float32 work on the bf16 matrix instructions: six products each, of 2516.6
-# TFLOP/s dense (a bare loop of them on random values holds 1815, a sixth of it
-# 302: the power limit).
+# TFLOP/s dense (a bare loop of them on random values holds 1750 - 1815, a sixth
+# of it 291 - 302: the power limit).
 PEAK_SPLIT_MFMA = 419.4
 PEAK_HBM = 8000.0        # GB/s
 

@@ -5,9 +5,10 @@
  * into three bf16 parts and six products accumulated in float32 (split.h),
  * the five small ones apart from the large one.
  *
- * What bounds it: the matrix cores and their power (61 % of the cycles busy
- * at the 1.9 GHz that the load leaves). An implicit GEMM of output channels x
- * pixels, 16 input channels of one tap an instruction step:
+ * What bounds it: the matrix cores and their power (busy 64 % of the CUs'
+ * busy cycles in the first layer below, vector instructions 9 %), then the
+ * barriers of the one block that a CU's LDS holds. An implicit GEMM of output
+ * channels x pixels, 16 input channels of one tap an instruction step:
  *  - a block computes 64 WM channels x 256 pixels, a wave 64 x 64 (two
  *    tiles each way: an operand read feeds two products of each kind);
  *  - the input patch of 16 channels is split once, by the thread that
@@ -29,8 +30,8 @@
  *
  * Measured on an MI355X against conv_mfma (conv.hip): 80 -> 129 channels at
  * 512 x 512 with normalisation (its 129th channel on conv_fewk_kernel both
- * times) 1207 -> 696 us, 256 -> 256 at 400 x 400 4187 -> 2237 us (125 -> 234
- * TFLOP/s), 96 -> 64 at 256 x 256 186 -> 133 us; error against 64-bit sums
+ * times) 1206 -> 702 us, 256 -> 256 at 400 x 400 4080 -> 2274 us (129 -> 231
+ * TFLOP/s), 96 -> 64 at 256 x 256 179 -> 127 us; error against 64-bit sums
  * 8.2e-7 -> 3.0e-7 on the first. 3 x 3 layers stay with Winograd: direct they
  * took 1.3 - 2.4 times as long (256 channels at 80 x 80, 64 at 320 x 320). */
 
@@ -52,10 +53,11 @@ static __device__ __forceinline__ __amdgpu_buffer_rsrc_t cs_rsrc(const float *p,
                                              0x00020000);
 }
 
-/* 16-byte operands of the filters, scaled as the input is (split.h): [64-channel block][16 input channels]
- * [tap][part][32-channel half][lane]. Lane l holds output channel l % 32 of
- * the half, input channels 8 (l / 32) .. + 7; zeros past K and C. One
- * thread per (block, slice, tap, half, lane). */
+/* 16-byte operands of the filters, scaled as the input is (split.h):
+ * [64-channel block][16 input channels][tap][part][32-channel half][lane].
+ * Lane l holds output channel l % 32 of the half, input channels 8 (l / 32)
+ * .. + 7; zeros past K and C. One thread per (block, slice, tap, half,
+ * lane). */
 __global__ void __launch_bounds__(256)
     conv_split_weights_kernel(const float *__restrict__ w, int K, int C, int nc,
                               split_u4 *__restrict__ wp, long long n)
@@ -443,8 +445,9 @@ conv_split_plan conv_split_choose(const conv_args &a, int ks, int st, int nb, in
      * median). Cut into about two blocks a CU instead, one layer in two ran 5 %
      * or more longer than it could, up to 1.6 times, and one in eight longer
      * than on conv_mfma, up to 1.9 times (19 -> 256 channels, normalised, at 38 x
-     * 470: 83 us there, 97 in two pieces, 72 whole); so cut, one in 20, layers of 17
-     * to 21 channels whose second slice is nearly empty, up to 1.4 times. */
+     * 470: 83 us there, 97 in two pieces, 72 whole); so cut, one in 20: most have
+     * 17 to 21 channels, whose second slice is nearly empty (up to 1.46 times), a
+     * few a nearly empty second round of blocks (up to 1.6 times). */
     const double slice = p.bm == 64 ? 14.4 + (a.mean ? 2.5 : 0.0) : 20.8 + (a.mean ? 1.4 : 0.0);
     const double mb = 8e-6 * nb * a.K * a.Ho * a.Wo / (p.bm == 64 ? 2.3 : 3.6);
     double best = 1e30;

@@ -8,13 +8,15 @@
  *
  * What bounds it: the matrix cores and the power they draw. Six bf16
  * products take 192 cycles where eight v_mfma_f32_32x32x2f32 take 512; on
- * random operands the bare instruction stream holds 1.81 PFLOP/s of bf16
- * (the clock falls from 2.4 to about 1.8 GHz), 302 TFLOP/s of float32
- * work, and a large bf16 library product 1.13 PFLOP/s. What the kernel
- * adds to the stream: 6.5 vector instructions a staged value for the split
- * and the LDS traffic of three parts, both in proportion to the tile's
- * sides, against matrix work in proportion to its area; hence the largest
- * tile that still gives the CUs equal shares.
+ * random operands the bare instruction stream holds 1.75 - 1.82 PFLOP/s of
+ * bf16 (2.48 on zeros: the clock falls), 291 - 302 TFLOP/s of float32 work,
+ * and a large bf16 library product 1.34 PFLOP/s. What the kernel adds to the
+ * stream: 6.5 vector instructions a staged value for the split and the LDS
+ * traffic of three parts, both in proportion to the tile's sides, against
+ * matrix work in proportion to its area; hence the largest tile that still
+ * gives the CUs equal shares. Of the CUs' busy cycles the matrix pipes take
+ * 0.57 and vector instructions 0.50 on the first shape below, 0.67 and 0.33
+ * on the second.
  *
  *  - A block stages 32 k of both operands: buffer loads through windows
  *    over the tile's rows (past the edge they read 0) into registers a
@@ -23,7 +25,8 @@
  *    A lane's MFMA operand is eight consecutive k: one ds_read_b128.
  *  - The 16-byte chunks of a row are stored XORed with bits of the row so
  *    that the 16 rows a quarter of a read touches lie in 64 different
- *    banks (without it 40 % of the LDS cycles were conflicts).
+ *    banks (conflicts take none of the LDS cycles with B N x K, 17 % with B
+ *    K x N).
  *  - The five products below hh have accumulators of their own, added to
  *    hh's at the end: added to the large sums one by one they round away
  *    (mm of a sum of squares did, which moved such sums by -1.3e-7 of their
@@ -34,9 +37,9 @@
  *    give them, at about the time of the fp32 kernel on top.
  *
  * Measured on an MI355X against the kernel on v_mfma_f32_32x32x2f32
- * (gemm.hip): 3202 x 4096 x 1024 with bias and GELU 238.5 -> 161.4 us (113 ->
- * 166 TFLOP/s of float32 work), 3202 x 1024 x 4096 232 -> 174 us, 1140 x
- * 11664 x 1140 (B given K x N) 265 -> 185 us; error against 64-bit sums at K
+ * (gemm.hip): 3202 x 4096 x 1024 with bias and GELU 241 -> 167 us (111 ->
+ * 161 TFLOP/s of float32 work), 3202 x 1024 x 4096 248 -> 179 us, 1140 x
+ * 11664 x 1140 (B given K x N) 291 -> 200 us; error against 64-bit sums at K
  * = 1024 6.4e-7 -> 2.1e-7. One block of a CU's two computes while the other
  * stages; 128 x 256 tiles of 4 x 64 x 128 waves ran 146 us on the first shape
  * with one accumulator set, but have no registers for two (199 us). */
@@ -475,7 +478,8 @@ struct split_cost {
     double alone, share, fixed, call, cut;
 };
 
-/* split_m, split_s and split_xs by how the operands come (split_row), fitted to 170000 times of 11600 products (M, N 16 .. 4096, K 513 .. 4096, every
+/* split_m, split_s and split_xs by how the operands come (split_row), fitted
+ * to 170000 times of 11600 products (M, N 16 .. 4096, K 513 .. 4096, every
  * tile and cut) on an MI355X: 16-byte rows within 2 - 3 % of them at the
  * median, 4-byte loads within 4 - 8 %. The gathered convolution, which is never
  * cut, has figures from the patch embedding. */

@@ -281,11 +281,11 @@ __device__ __forceinline__ double readlane_d(double v, int l)
  *    16 after its factor): within 16 rows in registers, below them on the
  *    matrix instructions.
  *  - All threads store factor and inverse in rows.
- * Bound by one wave's dependent chain, about 750 cycles a column pair. A
+ * Bound by one wave's dependent chain, about 710 cycles a column pair. A
  * block at n = 1600: 41 us with a whole-row sweep of the 64 columns (an LDS
- * round trip and up to 62 updates a lane each step), 22 us so, of 52k
- * cycles 7k the loads, 10k the look-ahead, 24k the factor, 11k the last rows
- * of the inverse, the stores and the release. */
+ * round trip and up to 62 updates a lane each step), 22 us so, of 54k
+ * cycles 7k the loads, 10k the look-ahead, 23k the factor, 14k the last rows
+ * of the inverse, the stores and the release (clock reads in a copy). */
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
     chol_diag_kernel(const double *__restrict__ A, double *__restrict__ L,
                       double *__restrict__ Linv, int n, int k, int nb,

@@ -414,27 +414,28 @@ __global__ void __launch_bounds__(64 * ATT_NW) attention_kernel(const att_args a
  * round away, all one way where the values have one sign (mean shift at 4000
  * keys -1.1e-8, so 3e-9; rms error at 128 keys, 32 channels 1.46e-7 against
  * the fp32 block's 1.05e-7, so 0.9e-7). With 64 channels these accumulators
- * would spill (160 us on the first shape below); there the small products of
- * 16 keys are summed apart and added once (155 us; of 32 keys 157). With 128,
- * adding so took 124 us for 8 heads, 1600 tokens, accumulators 110 (101 with
- * no sums apart).
+ * would spill (160 us for 2 x 16 heads, 1601 tokens); there the small products
+ * of 16 keys are summed apart and added once (155 us; of 32 keys 157; 147 with
+ * no sums apart). With 128, adding so took 124 us for 8 heads, 1600 tokens,
+ * accumulators 110 (101 with no sums apart).
  *
  * Per 32 keys, 32 queries and 64 channels 48 products (1536 cycles) run
  * beside 16 exponentials and 32 splits a lane (about 1200 cycles of vector
  * instructions): bound by those, by the loads' latency and by the two units
  * overlapping only between the 3 blocks that the registers hold. Measured on
- * an MI355X with the merge, against the fp32 block: 2 x 16 heads of 64, 1601
- * tokens 223 -> 147 us (143 TFLOP/s); 16 heads of 64, 785 tokens 56 -> 40;
- * 2 x 8 heads of 32, 400 tokens 18.7 -> 16; 2 x 16 heads of 32, 1601 tokens
- * 138 -> 88; 8 heads of 128, 1600 tokens 167 -> 95; 2 x 16 heads of 128, 2304
- * tokens 937 -> 595; 4 heads of 64, 49 tokens 12.2 -> 11.2. Tried: the next
- * tile's scores beside this one's softmax in one wave, 2 blocks a CU (64
- * channels 147 -> 155, 128 channels 596 -> 604). Error against 64 bits half
- * of the fp32 block's (4.1e-7, 8.4e-7: its 64 terms round each time). The
- * order of the blocks gave 188 -> 174 of those 147, loads without a range
- * check per value (rows past the keys read the last key again) the rest.
- * 65 .. 96 channels stay on the fp32 block: rows of 12 chunks would not
- * spread over the banks this way.
+ * one MI355X with the merge, against the fp32 block: 2 x 16 heads of 64, 1601
+ * tokens 230 -> 169 us (on another 224 -> 155, 136 TFLOP/s); 16 heads of 64,
+ * 785 tokens 59 -> 45; 2 x 8 heads of 32, 400 tokens 19.4 -> 17.2; 2 x 16 heads
+ * of 32, 1601 tokens 147 -> 99; 8 heads of 128, 1600 tokens 167 -> 109; 2 x 16
+ * heads of 128, 2304 tokens 937 -> 654; 4 heads of 64, 49 tokens 12.8 -> 12.4.
+ * Tried, before the sums apart: the next tile's scores beside this one's
+ * softmax in one wave, 2 blocks a CU (64 channels 147 -> 155, 128 channels 596
+ * -> 604). Error against 64 bits two fifths of the fp32 block's on the first
+ * shape (3.3e-7, 8.4e-7: its 64 terms round each time). The order of the
+ * blocks and loads without a range check per value (rows past the keys read
+ * the last key again) gave 188 -> 147 before the sums apart. 65 .. 96
+ * channels stay on the fp32 block: rows of 12 chunks would not spread over the
+ * banks this way.
  *
  * Values and probabilities are scaled as split.h says. Queries are scaled by
  * ATT_QUP and keys not: scores need absolute precision, and a query of 2^95
